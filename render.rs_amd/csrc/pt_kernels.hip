@@ -42,8 +42,7 @@ __global__ __launch_bounds__(kBlock) void raygen_kernel(PtSceneView S, PathBuffe
   const uint32_t all = total + N.ntrain;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     P.counts[0] = all;
-    P.counts[1] = 0;
-    P.counts[2] = 0;
+    *P.append() = 0;
     // N.counts[1] (training samples of the previous pass) is left alone: the
     // previous pass's optimiser steps may still be reading it, and this
     // pass's scan overwrites it before its own steps.
@@ -74,10 +73,9 @@ __global__ __launch_bounds__(kBlock) void raygen_kernel(PtSceneView S, PathBuffe
 
 __global__ void rotate_kernel(PathBuffers P) {
   P.stats[0] += P.counts[0];
-  P.stats[1] += P.counts[2];
-  P.counts[0] = P.counts[1];
-  P.counts[1] = 0;
-  P.counts[2] = 0;
+  P.stats[1] += P.counts[3];
+  P.counts[0] = P.counts[2];
+  *P.append() = 0;
 }
 
 __global__ __launch_bounds__(kBlock) void resolve_kernel(PathBuffers P, PtParams prm, double* __restrict__ accum) {
@@ -165,8 +163,7 @@ __global__ __launch_bounds__(kBlock) void raygen_batch_kernel(const PtJob* __res
                                                              uint32_t total) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     P.counts[0] = total;
-    P.counts[1] = 0;
-    P.counts[2] = 0;
+    *P.append() = 0;
   }
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x; slot < total; slot += stride) {
@@ -221,12 +218,15 @@ __global__ __launch_bounds__(kBlock) void shade_batch_kernel(const PtJob* __rest
       else
         shade_one<false, false>(J.S, P, J.prm, N, slot, cont, shadow, shadow2, se, query, so, nq, qbeta);
     }
-    if (P.srng)
-      push_shadow<true>(P, act, slot, shadow, so, shadow2, se);
-    else
-      push_shadow<false>(P, act, slot, shadow, so, shadow2, se);
-    const uint32_t nidx = wave_append(&P.counts[1], act && cont);
-    if (act && cont) qnext[nidx] = slot;
+    uint32_t nidx, sidx, qidx;
+    block_append<false>(P.append(), nullptr, cont, shadow || shadow2, false, nidx, sidx, qidx);
+    if (shadow || shadow2) {
+      if (P.srng)
+        put_shadow<true>(P, sidx, slot, shadow, so, shadow2, se);
+      else
+        put_shadow<false>(P, sidx, slot, shadow, so, shadow2, se);
+    }
+    if (cont) qnext[nidx] = slot;
   }
 }
 
@@ -234,7 +234,7 @@ template <bool QUAD>
 __global__ __launch_bounds__(kTraceBlock) void shadow_batch_kernel(const PtJob* __restrict__ jobs, PathBuffers P) {
   __shared__ uint32_t s_stack[kTraceStack * kTraceBlock];
   uint32_t* stk = s_stack + threadIdx.x;
-  const uint32_t n = P.counts[2];
+  const uint32_t n = P.counts[3];
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
     shadow_one<QUAD>(jobs[P.job[P.sq[i]]].S, P, i, stk);

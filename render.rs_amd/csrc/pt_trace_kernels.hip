@@ -40,7 +40,7 @@ template <int STACK, bool WALK, bool MOTION, int GEO, bool COUNT = false>
 __global__ __launch_bounds__(kTraceBlock) void shadow_kernel(PtSceneView S, PathBuffers P) {
   __shared__ uint32_t s_stack[STACK * kTraceBlock];
   uint32_t* stk = s_stack + threadIdx.x;
-  const uint32_t n = P.counts[2];
+  const uint32_t n = P.counts[3];
   const uint32_t stride = gridDim.x * blockDim.x;
   TraceCount tc;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)

@@ -342,7 +342,9 @@ struct PathBuffers {
   uint2* mstk;      // transparent scenes: each path's medium stack (8 x 8-bit medium indices)
   uint2* srng;      // transparent scenes: 64-bit seed of each shadow record's blocker walk
   float* stime;     // scenes with motion: shutter time of each shadow record (paths keep theirs in beta.w)
-  uint32_t* counts; // [0] live paths, [1] next live, [2] shadow rays, [3] unused
+  uint32_t* counts; // [0] live paths, [1] unused, [2] next live, [3] shadow records
+  // The append counters [2] (low half) and [3] as one word.
+  __device__ unsigned long long* append() const { return (unsigned long long*)(counts + 2); }
   unsigned long long* stats;  // [0] extension rays, [1] shadow rays, [2] cache queries, [3] training samples
   uint32_t* job;    // batches: job of each slot (null in sessions)
   uint32_t* qs;     // sorted-queue mode: the live queue grouped by shading class
