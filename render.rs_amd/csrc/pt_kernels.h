@@ -40,9 +40,14 @@ hipError_t pt_launch_bounce(const PtSceneView& S, const PathBuffers& P, const Pt
 // (extend), or the visibility of the shadow records. gt: trace blocks.
 hipError_t pt_launch_trace(const PtSceneView& S, const PathBuffers& P, const uint32_t* q, uint32_t gt, bool extend,
                            hipStream_t st);
-// The shading kernel of one bounce over the queue `qshade`.
-hipError_t pt_launch_shade(const PtSceneView& S, const PathBuffers& P, const PtParams& prm, const uint32_t* qshade,
-                           uint32_t* qnext, const NrcPathBuffers& N, uint32_t g, hipStream_t st);
+// The shading kernel of one bounce over the queue `qshade`, with
+// error-bounded ray origins or render.rs's fixed push (S.ray_offset > 0).
+hipError_t pt_launch_shade_bounded(const PtSceneView& S, const PathBuffers& P, const PtParams& prm,
+                                   const uint32_t* qshade, uint32_t* qnext, const NrcPathBuffers& N, uint32_t g,
+                                   hipStream_t st);
+hipError_t pt_launch_shade_fixed(const PtSceneView& S, const PathBuffers& P, const PtParams& prm,
+                                 const uint32_t* qshade, uint32_t* qnext, const NrcPathBuffers& N, uint32_t g,
+                                 hipStream_t st);
 // One pass of a batch: raygen over every job's slots (jobs sorted by
 // slot_begin and pix_begin), `bounces` rounds of extend / shade / shadow
 // with each path reading its own job's scene and parameters, and the

@@ -347,7 +347,8 @@ hipError_t pt_launch_bounce(const PtSceneView& S, const PathBuffers& P, const Pt
     hipLaunchKernelGGL(sort_scatter_kernel, dim3(kSortBlocks), dim3(kBlock), 0, st, S, P, q);
     qshade = P.qs;
   }
-  e = pt_launch_shade(S, P, prm, qshade, qnext, N, g, st);
+  e = S.ray_offset > 0.f ? pt_launch_shade_fixed(S, P, prm, qshade, qnext, N, g, st)
+                         : pt_launch_shade_bounded(S, P, prm, qshade, qnext, N, g, st);
   if (e != hipSuccess) return e;
   if (ev) (void)hipEventRecord(ev[2], st);
   e = pt_launch_trace(S, P, nullptr, gt, false, st);

@@ -1,0 +1,12 @@
+// Shading kernels with error-bounded ray origins.
+#include "pt_shade.h"
+
+namespace rrhip {
+
+hipError_t pt_launch_shade_bounded(const PtSceneView& S, const PathBuffers& P, const PtParams& prm,
+                                const uint32_t* qshade, uint32_t* qnext, const NrcPathBuffers& N, uint32_t g,
+                                hipStream_t st) {
+  return launch_shade<false>(S, P, prm, qshade, qnext, N, g, st);
+}
+
+}  // namespace rrhip

@@ -380,7 +380,10 @@ __device__ __forceinline__ bool sample_light(const PtSceneView& S, const PtLight
 // spread beyond one pixel in d.w, its width in prev.w, pt/mod.rs:477-480),
 // and a hit on such a material shades with the fields its patterns give
 // there (pt/mod.rs:685-689, 389-440).
-template <bool NRC, bool TR, bool FILM = false, bool FIXED = false, bool HAIR = false, bool PAT = false>
+// MEDIA: the scene has an atmosphere or interior media (caches are never
+// attached to scenes with media).
+template <bool NRC, bool TR, bool FILM = false, bool FIXED = false, bool HAIR = false, bool PAT = false,
+          bool MEDIA = !NRC>
 __device__ __forceinline__ void shade_one(const PtSceneView& S, const PathBuffers& P, const PtParams& prm,
                                           const NrcPathBuffers& N, uint32_t slot, bool& cont, bool& shadow,
                                           bool& shadow2, ShadowOut& se, bool& query, ShadowOut& so, NrcQuery& nq,
@@ -419,7 +422,7 @@ __device__ __forceinline__ void shade_one(const PtSceneView& S, const PathBuffer
       sdepth = (flags >> kStackShift) & 0xFu;
       skips = (flags >> kSkipShift) & 0x1Fu;
     }
-    const int cur = NRC ? -1 : stack_top(mst, sdepth, S.atmosphere);  // the segment's medium
+    const int cur = MEDIA ? stack_top(mst, sdepth, S.atmosphere) : -1;  // the segment's medium
     // Film: radiance of this path that goes to the diffuse AOV (all of it
     // until a first continuation is sampled specular-like); aux_set: the
     // first real hit is recorded; travel: distance to it so far.
@@ -447,7 +450,7 @@ __device__ __forceinline__ void shade_one(const PtSceneView& S, const PathBuffer
     // equiangular strategy for point lights) and an HG continuation
     // instead of the surface.
     bool in_medium = false, absorbed = false;
-    if (!NRC && cur >= 0) {  // caches are never attached to scenes with media
+    if (MEDIA && cur >= 0) {
       const PtMedium& md = S.media[cur];
       const float t_limit = hn.w < 0.f ? 1e8f : hn.w;
       const float t_seg = fminf(t_limit, md.max_distance);
@@ -613,7 +616,7 @@ __device__ __forceinline__ void shade_one(const PtSceneView& S, const PathBuffer
       // the ray continues unchanged past the surface
     } else if (hn.w >= 0.f && !in_medium && !absorbed) {
       const uint32_t hm = P.hit_m[slot];
-      const PtMaterial m = PAT ? mres : S.materials[hm & 0x7FFFFFFFu];
+      const PtMaterial& m = PAT ? mres : S.materials[hm & 0x7FFFFFFFu];
       const bool entering = (hm >> 31) != 0;
       const V3 p = hit_point();
       const V3 ng = v3(hn.x, hn.y, hn.z);
@@ -652,7 +655,7 @@ __device__ __forceinline__ void shade_one(const PtSceneView& S, const PathBuffer
                                         so)) {
                 so.c = beta * so.c;
                 so.medium = cur;
-                if (!NRC && cur >= 0 && !walk)
+                if (MEDIA && cur >= 0 && !walk)
                   so.c = so.c * medium_transmittance(S.media[cur], so.o, so.d, so.tmax, rng);
                 shadow = maxc(so.c) > 0.f;
               }
@@ -752,7 +755,7 @@ __device__ __forceinline__ void shade_one(const PtSceneView& S, const PathBuffer
             so.medium = cur;
             // shadow rays through a medium carry its transmittance (or
             // pick it up on their blocker walk)
-            if (!NRC && cur >= 0 && !walk)
+            if (MEDIA && cur >= 0 && !walk)
               so.c = so.c * medium_transmittance(S.media[cur], so.o, so.d, so.tmax, rng);
             shadow = maxc(so.c) > 0.f;
           }
@@ -837,7 +840,7 @@ __device__ __forceinline__ void put_shadow(const PathBuffers& P, uint32_t idx, u
 
 // The shade pass over the queue q: each path's step, then the block-wide
 // append of its shadow records, continuation and cache query.
-template <bool NRC, bool TR, bool FILM, bool FIXED, bool HAIR, bool PAT = false>
+template <bool NRC, bool TR, bool MEDIA, bool FILM, bool FIXED, bool HAIR, bool PAT = false>
 __device__ __forceinline__ void shade_pass(const PtSceneView& S, const PathBuffers& P, const PtParams& prm,
                                            const uint32_t* __restrict__ q, uint32_t* __restrict__ qnext,
                                            const NrcPathBuffers& N) {
@@ -854,8 +857,8 @@ __device__ __forceinline__ void shade_pass(const PtSceneView& S, const PathBuffe
     uint32_t slot = 0;
     if (act) {
       slot = q[i];
-      shade_one<NRC, TR, FILM, FIXED, HAIR, PAT>(S, P, prm, N, slot, cont, shadow, shadow2, se, query, so, nq,
-                                                 qbeta);
+      shade_one<NRC, TR, FILM, FIXED, HAIR, PAT, MEDIA>(S, P, prm, N, slot, cont, shadow, shadow2, se, query, so,
+                                                        nq, qbeta);
     }
     uint32_t nidx, sidx, qidx;
     block_append<NRC>(P.append(), NRC ? &N.counts[0] : nullptr, cont, shadow || shadow2, query, nidx, sidx, qidx);
