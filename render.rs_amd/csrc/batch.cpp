@@ -212,7 +212,7 @@ int rrhip_batch_create(rrhip_ctx* ctx, uint32_t num_jobs, const rrhip_batch_job*
   }
   if (e == hipSuccess && motion) e = alloc_n(b, &P.stime, n);
   if (e == hipSuccess) e = alloc_n(b, &P.job, n);
-  if (e == hipSuccess) e = alloc_n(b, &P.counts, 8);
+  if (e == hipSuccess) e = alloc_n(b, &P.rounds, kRoundWords);
   if (e == hipSuccess) e = alloc_n(b, &P.stats, 4);
   // The whole schedule's job tables, uploaded once.
   if (e == hipSuccess) {

@@ -27,18 +27,25 @@ hipError_t pt_launch_raygen(const PtSceneView& S, const PathBuffers& P, const Pt
                             uint32_t total, const NrcPathBuffers& N, const uint64_t* sample0_dev, hipStream_t st);
 // *dst = v, in stream order (a kernel, so it never becomes a memset node).
 hipError_t pt_launch_set_u64(uint64_t* dst, uint64_t v, hipStream_t st);
-// One bounce over the live queue `q`: closest hit, shading (emission + MIS,
-// NEE shadow rays, BSDF continuation, Russian roulette) into `qnext`,
-// shadow rays, counter rotation. `capacity` bounds every queue. With
-// N.q set, paths terminate into radiance-cache queries (see NrcPathBuffers).
+// Bounce round P.round over the live queue `q`: closest hit, shading
+// (emission + MIS, NEE shadow rays, BSDF continuation, Russian roulette)
+// into `qnext`, shadow rays. In opaque scenes the shadow rays of a round
+// are traced with the next round's closest hits, or after the last round by
+// pt_launch_last_shadows. `capacity` bounds every queue. With N.q set,
+// paths terminate into radiance-cache queries (see NrcPathBuffers).
 // ev (profiling, may be null): four events recorded before extend, before
 // shade (the queue sort included), before shadow, and after it.
 hipError_t pt_launch_bounce(const PtSceneView& S, const PathBuffers& P, const PtParams& prm,
                             const uint32_t* q, uint32_t* qnext, uint32_t capacity, const NrcPathBuffers& N,
                             hipStream_t st, const hipEvent_t* ev = nullptr);
-// The trace kernels of one bounce: closest hits of the live queue `q`
-// (extend), or the visibility of the shadow records. gt: trace blocks.
-hipError_t pt_launch_trace(const PtSceneView& S, const PathBuffers& P, const uint32_t* q, uint32_t gt, bool extend,
+// The shadow rays of the last round (P.round = the number of rounds).
+hipError_t pt_launch_last_shadows(const PtSceneView& S, const PathBuffers& P, uint32_t capacity, hipStream_t st);
+// The trace kernels, with gt blocks: closest hits of the live queue `q` of
+// P.round (kTraceExtend), visibility of the shadow records that the round
+// before wrote (kTraceShadow), or both in one launch (kTraceRound: opaque
+// scenes, not while profiling).
+enum TraceWork { kTraceExtend, kTraceShadow, kTraceRound };
+hipError_t pt_launch_trace(const PtSceneView& S, const PathBuffers& P, const uint32_t* q, uint32_t gt, TraceWork work,
                            hipStream_t st);
 // The shading kernel of one bounce over the queue `qshade`, with
 // error-bounded ray origins or render.rs's fixed push (S.ray_offset > 0).
@@ -53,7 +60,7 @@ hipError_t pt_launch_shade_fixed(const PtSceneView& S, const PathBuffers& P, con
 // with each path reading its own job's scene and parameters, and the
 // resolve of every job's pixels into its accumulator. `quadrics`: some
 // job's scene holds quadrics (the trace kernels then carry their solvers).
-hipError_t pt_launch_batch_pass(const PtJob* jobs, uint32_t nj, const PathBuffers& P, uint32_t total,
+hipError_t pt_launch_batch_pass(const PtJob* jobs, uint32_t nj, PathBuffers P, uint32_t total,
                                  uint32_t total_pix, uint32_t bounces, bool quadrics, hipStream_t st);
 // Every job of a batch in one persistent launch: `lanes` path slots (a
 // multiple of the block), each pulling (job, pixel) items from *next_item

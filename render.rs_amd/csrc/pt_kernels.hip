@@ -16,6 +16,8 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "pt_wave.h"
 
 namespace rrhip {
@@ -34,15 +36,19 @@ __global__ __launch_bounds__(kBlock) void pcg32_draws_kernel(const uint64_t* __r
   for (uint32_t k = 0; k < count; k++) out[(size_t)i * count + k] = rng.next_u32();
 }
 
+// The round words of a pass that starts with n paths.
+__device__ __forceinline__ void start_rounds(const PathBuffers& P, uint32_t n) {
+  for (uint32_t i = threadIdx.x; i < kRoundWords; i += blockDim.x) P.rounds[i] = i == 0 ? n : 0;
+}
+
 // sample0_dev (when set) supplies the pass's first sample index from device
 // memory, so a captured pass graph can be replayed for any sample range.
 __global__ __launch_bounds__(kBlock) void raygen_kernel(PtSceneView S, PathBuffers P, PtParams prm, uint32_t total,
                                                        NrcPathBuffers N, const uint64_t* __restrict__ sample0_dev) {
   if (sample0_dev) prm.sample0 = *sample0_dev;
   const uint32_t all = total + N.ntrain;
+  if (blockIdx.x == 0) start_rounds(P, all);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    P.counts[0] = all;
-    *P.append() = 0;
     // N.counts[1] (training samples of the previous pass) is left alone: the
     // previous pass's optimiser steps may still be reading it, and this
     // pass's scan overwrites it before its own steps.
@@ -71,14 +77,17 @@ __global__ __launch_bounds__(kBlock) void raygen_kernel(PtSceneView S, PathBuffe
   }
 }
 
-__global__ void rotate_kernel(PathBuffers P) {
-  P.stats[0] += P.counts[0];
-  P.stats[1] += P.counts[3];
-  P.counts[0] = P.counts[2];
-  *P.append() = 0;
+// Adds the rays of rounds [0, P.round) to the session's totals.
+__device__ __forceinline__ void add_ray_totals(const PathBuffers& P) {
+  for (uint32_t i = threadIdx.x; i <= P.round; i += blockDim.x) {
+    const unsigned long long w = P.rounds[i];
+    if (i < P.round && (uint32_t)w) atomicAdd(P.stats + 0, (unsigned long long)(uint32_t)w);
+    if (w >> 32) atomicAdd(P.stats + 1, w >> 32);
+  }
 }
 
 __global__ __launch_bounds__(kBlock) void resolve_kernel(PathBuffers P, PtParams prm, double* __restrict__ accum) {
+  if (blockIdx.x == 0) add_ray_totals(P);
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < prm.npix; c += stride) resolve_one(P, prm, accum, c, 0);
 }
@@ -161,10 +170,7 @@ __global__ __launch_bounds__(kBlock) void resolve_film_kernel(PathBuffers P, PtP
 
 __global__ __launch_bounds__(kBlock) void raygen_batch_kernel(const PtJob* __restrict__ jobs, uint32_t nj, PathBuffers P,
                                                              uint32_t total) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    P.counts[0] = total;
-    *P.append() = 0;
-  }
+  if (blockIdx.x == 0) start_rounds(P, total);
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x; slot < total; slot += stride) {
     const uint32_t j = find_job<false>(jobs, nj, slot);
@@ -180,7 +186,7 @@ __global__ __launch_bounds__(kTraceBlock) void extend_batch_kernel(const PtJob* 
                                                                   const uint32_t* __restrict__ q) {
   __shared__ uint32_t s_stack[kTraceStack * kTraceBlock];
   uint32_t* stk = s_stack + threadIdx.x;
-  const uint32_t n = P.counts[0];
+  const uint32_t n = P.live();
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     const uint32_t slot = q[i];
@@ -194,7 +200,7 @@ __global__ __launch_bounds__(kTraceBlock) void extend_batch_kernel(const PtJob* 
 
 __global__ __launch_bounds__(kBlock) void shade_batch_kernel(const PtJob* __restrict__ jobs, PathBuffers P,
                                                             const uint32_t* __restrict__ q, uint32_t* __restrict__ qnext) {
-  const uint32_t n = P.counts[0];
+  const uint32_t n = P.live();
   const uint32_t stride = gridDim.x * blockDim.x;
   const NrcPathBuffers N{};
   for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
@@ -234,7 +240,7 @@ template <bool QUAD>
 __global__ __launch_bounds__(kTraceBlock) void shadow_batch_kernel(const PtJob* __restrict__ jobs, PathBuffers P) {
   __shared__ uint32_t s_stack[kTraceStack * kTraceBlock];
   uint32_t* stk = s_stack + threadIdx.x;
-  const uint32_t n = P.counts[3];
+  const uint32_t n = P.shadows();
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
     shadow_one<QUAD>(jobs[P.job[P.sq[i]]].S, P, i, stk);
@@ -242,6 +248,7 @@ __global__ __launch_bounds__(kTraceBlock) void shadow_batch_kernel(const PtJob* 
 
 __global__ __launch_bounds__(kBlock) void resolve_batch_kernel(const PtJob* __restrict__ jobs, uint32_t nj, PathBuffers P,
                                                               uint32_t total_pix) {
+  if (blockIdx.x == 0) add_ray_totals(P);
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < total_pix; g += stride) {
     const PtJob& J = jobs[find_job<true>(jobs, nj, g)];
@@ -272,7 +279,7 @@ __global__ __launch_bounds__(kBlock) void sort_count_kernel(PtSceneView S, PathB
   for (uint32_t i = threadIdx.x; i < kSortKeys; i += blockDim.x) h[i] = 0;
   __syncthreads();
   uint32_t b0, b1;
-  block_range(P.counts[0], b0, b1);
+  block_range(P.live(), b0, b1);
   for (uint32_t i = b0 + threadIdx.x; i < b1; i += blockDim.x) atomicAdd(&h[sort_key(S, P, q[i])], 1u);
   __syncthreads();
   for (uint32_t k = threadIdx.x; k < kSortKeys; k += blockDim.x) P.sort_hist[k * kSortBlocks + blockIdx.x] = h[k];
@@ -308,7 +315,7 @@ __global__ __launch_bounds__(kBlock) void sort_scatter_kernel(PtSceneView S, Pat
   for (uint32_t k = threadIdx.x; k < kSortKeys; k += blockDim.x) cur[k] = P.sort_hist[k * kSortBlocks + blockIdx.x];
   __syncthreads();
   uint32_t b0, b1;
-  block_range(P.counts[0], b0, b1);
+  block_range(P.live(), b0, b1);
   for (uint32_t i = b0 + threadIdx.x; i < b1; i += blockDim.x) {
     const uint32_t slot = q[i];
     P.qs[atomicAdd(&cur[sort_key(S, P, slot)], 1u)] = slot;
@@ -331,13 +338,23 @@ hipError_t pt_launch_set_u64(uint64_t* dst, uint64_t v, hipStream_t st) {
   return hipGetLastError();
 }
 
+// Trace launches have a block per 128 queue entries, as far as the capacity
+// tells: blocks beyond the live paths end at once, and the dispatcher
+// balances rays of very different length better than 4,096 striding blocks
+// did (540p instanced field, 8 samples: frame 20.2 -> 18.6 ms).
+static uint32_t trace_grid(uint64_t capacity) {
+  const uint64_t b = (capacity + kTraceBlock - 1) / kTraceBlock;
+  return (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(1, b));
+}
+
 hipError_t pt_launch_bounce(const PtSceneView& S, const PathBuffers& P, const PtParams& prm, const uint32_t* q,
                             uint32_t* qnext, uint32_t capacity, const NrcPathBuffers& N, hipStream_t st,
                             const hipEvent_t* ev) {
   const uint32_t g = grid_for(capacity);
-  const uint32_t gt = grid_for(capacity, kTraceBlock);
+  const uint32_t gt = trace_grid(capacity);
+  const bool merged = !P.prof && !S.transparent;
   if (ev) (void)hipEventRecord(ev[0], st);
-  hipError_t e = pt_launch_trace(S, P, q, gt, true, st);
+  hipError_t e = pt_launch_trace(S, P, q, gt, merged ? kTraceRound : kTraceExtend, st);
   if (e != hipSuccess) return e;
   if (ev) (void)hipEventRecord(ev[1], st);
   const uint32_t* qshade = q;
@@ -351,19 +368,28 @@ hipError_t pt_launch_bounce(const PtSceneView& S, const PathBuffers& P, const Pt
                          : pt_launch_shade_bounded(S, P, prm, qshade, qnext, N, g, st);
   if (e != hipSuccess) return e;
   if (ev) (void)hipEventRecord(ev[2], st);
-  e = pt_launch_trace(S, P, nullptr, gt, false, st);
-  if (e != hipSuccess) return e;
+  if (!merged) {
+    PathBuffers Q = P;
+    Q.round = P.round + 1;  // the records this round wrote
+    e = pt_launch_trace(S, Q, nullptr, gt, kTraceShadow, st);
+    if (e != hipSuccess) return e;
+  }
   if (ev) (void)hipEventRecord(ev[3], st);
-  hipLaunchKernelGGL(rotate_kernel, dim3(1), dim3(1), 0, st, P);
   return hipGetLastError();
 }
 
-hipError_t pt_launch_batch_pass(const PtJob* jobs, uint32_t nj, const PathBuffers& P, uint32_t total,
+hipError_t pt_launch_last_shadows(const PtSceneView& S, const PathBuffers& P, uint32_t capacity, hipStream_t st) {
+  if (P.prof || S.transparent) return hipSuccess;
+  return pt_launch_trace(S, P, nullptr, trace_grid(capacity), kTraceRound, st);
+}
+
+hipError_t pt_launch_batch_pass(const PtJob* jobs, uint32_t nj, PathBuffers P, uint32_t total,
                                  uint32_t total_pix, uint32_t bounces, bool quadrics, hipStream_t st) {
   const uint32_t g = grid_for(total);
-  const uint32_t gt = grid_for(total, kTraceBlock);
+  const uint32_t gt = trace_grid(total);
   hipLaunchKernelGGL(raygen_batch_kernel, dim3(g), dim3(kBlock), 0, st, jobs, nj, P, total);
   for (uint32_t b = 0; b < bounces; b++) {
+    P.round = b;
     const uint32_t* q = (b & 1) ? P.q1 : P.q0;
     uint32_t* qn = (b & 1) ? P.q0 : P.q1;
     if (quadrics)
@@ -371,11 +397,11 @@ hipError_t pt_launch_batch_pass(const PtJob* jobs, uint32_t nj, const PathBuffer
     else
       hipLaunchKernelGGL(extend_batch_kernel<false>, dim3(gt), dim3(kTraceBlock), 0, st, jobs, P, q);
     hipLaunchKernelGGL(shade_batch_kernel, dim3(g), dim3(kBlock), 0, st, jobs, P, q, qn);
+    P.round = b + 1;  // the records this round wrote
     if (quadrics)
       hipLaunchKernelGGL(shadow_batch_kernel<true>, dim3(gt), dim3(kTraceBlock), 0, st, jobs, P);
     else
       hipLaunchKernelGGL(shadow_batch_kernel<false>, dim3(gt), dim3(kTraceBlock), 0, st, jobs, P);
-    hipLaunchKernelGGL(rotate_kernel, dim3(1), dim3(1), 0, st, P);
   }
   hipLaunchKernelGGL(resolve_batch_kernel, dim3(grid_for(total_pix)), dim3(kBlock), 0, st, jobs, nj, P, total_pix);
   return hipGetLastError();

@@ -167,7 +167,7 @@ hipError_t alloc_paths(rrhip_session* s, uint64_t n) {
     if (e == hipSuccess) e = alloc_in(m, &P.aux1, n);
     if (e == hipSuccess) e = alloc_in(m, &P.aux_id, n);
   }
-  if (e == hipSuccess) e = alloc_in(m, &P.counts, 4);
+  if (e == hipSuccess) e = alloc_in(m, &P.rounds, kRoundWords);
   if (e == hipSuccess) s->path_cap = n;
   return e;
 }
@@ -277,8 +277,11 @@ hipError_t enqueue_pass(rrhip_session* s, uint32_t n, uint32_t ncol, const uint3
   for (uint32_t b = 0; b < rounds && e == hipSuccess; b++) {
     const uint32_t* q = (b & 1) ? P.q1 : P.q0;
     uint32_t* qn = (b & 1) ? P.q0 : P.q1;
+    P.round = b;
     e = pt_launch_bounce(s->S, P, prm, q, qn, paths, N, st, prof ? ev + 4 * b : nullptr);
   }
+  P.round = rounds;
+  if (e == hipSuccess) e = pt_launch_last_shadows(s->S, P, paths, st);
   hipEvent_t* ev_nrc = prof ? ev + 4 * rounds : nullptr;
   bool nrc_timed = false, steps_timed = false;
   hipStream_t ts_used = st;
@@ -323,7 +326,7 @@ hipError_t enqueue_pass(rrhip_session* s, uint32_t n, uint32_t ncol, const uint3
       nrc->pending = e == hipSuccess;
     }
   }
-  if (e == hipSuccess) e = pt_launch_resolve(s->P, prm, s->d_accum, s->film ? s->d_film : nullptr, st);
+  if (e == hipSuccess) e = pt_launch_resolve(P, prm, s->d_accum, s->film ? s->d_film : nullptr, st);
   if (prof && e == hipSuccess) {
     // wait for the pass (and its optimiser steps) and sum the kernel times
     e = hipStreamSynchronize(st);

@@ -312,6 +312,9 @@ struct PtSceneView {
   PtCamera cam;
 };
 
+// Bounce rounds of a pass are at most 255 + 16 (bounces and pass-throughs).
+constexpr uint32_t kRoundWords = 255 + 16 + 2;
+
 // Wavefront path state, structure of arrays over path slots.
 struct PathBuffers {
   float4* o;        // origin.xyz, prev_pdf
@@ -342,9 +345,14 @@ struct PathBuffers {
   uint2* mstk;      // transparent scenes: each path's medium stack (8 x 8-bit medium indices)
   uint2* srng;      // transparent scenes: 64-bit seed of each shadow record's blocker walk
   float* stime;     // scenes with motion: shutter time of each shadow record (paths keep theirs in beta.w)
-  uint32_t* counts; // [0] live paths, [1] unused, [2] next live, [3] shadow records
-  // The append counters [2] (low half) and [3] as one word.
-  __device__ unsigned long long* append() const { return (unsigned long long*)(counts + 2); }
+  // Word r: paths that enter bounce round r (low half) and shadow records
+  // that round r - 1 wrote (high half); kRoundWords of them, cleared by
+  // raygen, so no launch is needed between rounds.
+  unsigned long long* rounds;
+  uint32_t round;   // the round a launch works on (set by the host for each launch)
+  __device__ uint32_t live() const { return (uint32_t)rounds[round]; }
+  __device__ uint32_t shadows() const { return (uint32_t)(rounds[round] >> 32); }
+  __device__ unsigned long long* append() const { return rounds + round + 1; }
   unsigned long long* stats;  // [0] extension rays, [1] shadow rays, [2] cache queries, [3] training samples
   uint32_t* job;    // batches: job of each slot (null in sessions)
   uint32_t* qs;     // sorted-queue mode: the live queue grouped by shading class
