@@ -14,6 +14,10 @@ constexpr uint32_t kPtTraceStack = 48;
 // samples whose id found no slot [19].
 constexpr uint32_t kFilmIds = 4;
 constexpr uint32_t kFilmStride = 12 + 2 * kFilmIds;
+constexpr uint32_t kFilmChannels = 18;  // RRHIP_FILM_CHANNELS
+// Pixels whose channels one launch of the film read-back makes: 38 MB of
+// device memory, however large the film is.
+constexpr uint32_t kFilmImageRows = 1u << 18;
 // Hull crossings and cutout pass-throughs per path (pt/mod.rs:32): they do
 // not count as bounces, so transparent scenes run this many extra rounds.
 constexpr uint32_t kPtMaxSkips = 16;
@@ -98,6 +102,9 @@ hipError_t pt_launch_relmse(const double* accum, const double* ref_accum, uint32
 // doubles into `partial`); the caller adds them.
 hipError_t pt_launch_count_sum(const double* accum, uint32_t npix, double* partial, uint32_t blocks,
                                hipStream_t st);
+// The film's channels (npix x kFilmChannels doubles into `out`) from the
+// accumulators.
+hipError_t pt_launch_film_image(const double* accum, const double* film, uint32_t npix, double* out, hipStream_t st);
 // Adaptive sampling: the pixels of live list `in` (n columns; null: pixel
 // = column) whose accumulators have not met the stopping rule of
 // pt/mod.rs:319-325 at tolerance `tol`, in column order, into `out`; their

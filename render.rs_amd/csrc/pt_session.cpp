@@ -65,6 +65,7 @@ struct rrhip_session {
   // accumulator (kFilmStride doubles per pixel) here.
   bool film = false;
   double* d_film = nullptr;
+  double* d_film_image = nullptr;  // channels of kFilmImageRows pixels, allocated by the first read
   // Profiling (rrhip_session_set_profiling): counting trace kernels whose
   // fetch totals land in prof_counts, events around each bounce's kernels
   // and the cache's inference and optimiser steps, device times summed per
@@ -119,6 +120,7 @@ void free_session(rrhip_session* s) {
   free_profile_events(s);
   if (s->prof_counts) (void)hipFree(s->prof_counts);
   if (s->d_film) (void)hipFree(s->d_film);
+  if (s->d_film_image) (void)hipFree(s->d_film_image);
   for (void* p : s->mem) (void)hipFree(p);
   s->mem.clear();
   delete s;
@@ -537,9 +539,9 @@ int rrhip_session_set_film(rrhip_session* s, int enable) {
   RRHIP_HIP_TRY(hipSetDevice(s->scene->ctx->device));
   RRHIP_HIP_TRY(hipStreamSynchronize(s->scene->ctx->stream));
   drop_graphs(s);  // captured passes hold the old buffers
-  if (s->d_film) {
-    (void)hipFree(s->d_film);
-    s->d_film = nullptr;
+  for (double** p : {&s->d_film, &s->d_film_image}) {
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
   }
   s->film = enable != 0;
   hipError_t e = alloc_paths(s, s->path_cap);
@@ -564,37 +566,17 @@ int rrhip_read_film(rrhip_session* s, double* out) {
   if (!out) return fail(RRHIP_ERR_INVALID_ARGUMENT, "rrhip_read_film: null output");
   if (!s->film) return fail(RRHIP_ERR_INVALID_ARGUMENT, "rrhip_read_film: film mode is off");
   RRHIP_HIP_TRY(hipSetDevice(s->scene->ctx->device));
-  const uint64_t npix = s->prm.npix;
-  std::vector<double> acc(npix * RRHIP_ACCUM_STRIDE), film(npix * kFilmStride);
+  static_assert(kFilmChannels == RRHIP_FILM_CHANNELS, "film channels");
+  const uint32_t npix = s->prm.npix, rows = std::min(npix, kFilmImageRows);
   hipStream_t st = s->scene->ctx->stream;
-  RRHIP_HIP_TRY(hipMemcpyAsync(acc.data(), s->d_accum, acc.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-  RRHIP_HIP_TRY(hipMemcpyAsync(film.data(), s->d_film, film.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-  RRHIP_HIP_TRY(hipStreamSynchronize(st));
-  // pt/mod.rs:223-274: sample means; specular = max(beauty - diffuse, 0);
-  // depth over the samples with a first real hit; the most voted id (the
-  // first of equal counts) and its share of the samples.
-  for (uint64_t p = 0; p < npix; p++) {
-    const double* a = &acc[p * RRHIP_ACCUM_STRIDE];
-    const double* f = &film[p * kFilmStride];
-    double* o = out + p * RRHIP_FILM_CHANNELS;
-    const double n = a[6] > 0.0 ? a[6] : 1.0;
-    for (int c = 0; c < 3; c++) {
-      o[c] = a[c] / n;
-      o[3 + c] = f[c] / n;
-      o[6 + c] = std::max(o[c] - o[3 + c], 0.0);
-      o[9 + c] = f[3 + c] / n;
-      o[12 + c] = f[6 + c] / n;
-    }
-    o[15] = f[10] > 0.0 ? f[9] / f[10] : 0.0;
-    double best_id = 0.0, best_n = 0.0;
-    for (uint32_t j = 0; j < kFilmIds; j++) {
-      if (f[11 + kFilmIds + j] > best_n) {
-        best_n = f[11 + kFilmIds + j];
-        best_id = f[11 + j];
-      }
-    }
-    o[16] = best_id;
-    o[17] = best_n / n;
+  if (!s->d_film_image) RRHIP_HIP_TRY(hipMalloc((void**)&s->d_film_image, (uint64_t)rows * kFilmChannels * sizeof(double)));
+  for (uint32_t p = 0; p < npix; p += rows) {
+    const uint32_t n = std::min(rows, npix - p);
+    RRHIP_HIP_TRY(pt_launch_film_image(s->d_accum + (uint64_t)p * RRHIP_ACCUM_STRIDE, s->d_film + (uint64_t)p * kFilmStride,
+                                       n, s->d_film_image, st));
+    RRHIP_HIP_TRY(hipMemcpyAsync(out + (uint64_t)p * kFilmChannels, s->d_film_image,
+                                 (uint64_t)n * kFilmChannels * sizeof(double), hipMemcpyDeviceToHost, st));
+    RRHIP_HIP_TRY(hipStreamSynchronize(st));
   }
   return RRHIP_OK;
 }
