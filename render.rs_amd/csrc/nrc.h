@@ -61,7 +61,7 @@ struct NrcControl {
   uint32_t n;        // samples in the pending batch
   uint32_t step;     // optimiser steps taken
   float last_loss;   // loss of the last batch
-  uint32_t pad;
+  uint32_t t;        // number of the step being run (step + 1, set by its first launch)
 };
 
 // y (n x 3 floats) for n queries (count read from `count` when non-null).
@@ -73,19 +73,24 @@ hipError_t nrc_launch_infer_paths(const NrcGridView& G, const NrcQuery* q, const
                                   hipStream_t st);
 // Forward + backward over the batch (ctl->n samples, <= capacity): block
 // partials into `part`, each sample's 32 encoding gradients into `genc`
-// (capacity x 32 floats), then the grid gradients into `grid_grad`.
-hipError_t nrc_launch_train(const NrcGridView& G, const NrcQuery* q, const float* targets,
-                            const NrcControl* ctl, uint32_t capacity, float* part, float* genc,
-                            unsigned long long* grid_grad, hipStream_t st);
+// (capacity x 32 floats), then the grid gradients into `grid_grad`, marking
+// in `touched` (a byte per 4 parameters) where one waits.
+hipError_t nrc_launch_train(const NrcGridView& G, const NrcQuery* q, const float* targets, NrcControl* ctl,
+                            uint32_t capacity, float* part, float* genc, unsigned long long* grid_grad,
+                            uint8_t* touched, hipStream_t st);
+// The rest of a step without a moving average: MLP reduction, Adam on the
+// MLP and the grid, the bf16 copies, the step count; clears the gradients.
+hipError_t nrc_launch_update(const NrcGridView& G, const float* part, NrcControl* ctl, float* w, float* wm, float* wv,
+                             uint16_t* wf, uint16_t* wb, float* table, float* m, float* v,
+                             unsigned long long* grid_grad, uint8_t* touched, NrcHyper hp, hipStream_t st);
 // Sums the partials; with `apply`, Adam on the MLP master weights (step
-// ctl->step + 1), else the summed gradient into `grad_out`; loss into ctl.
+// ctl->t), else the summed gradient into `grad_out`; loss into ctl.
 hipError_t nrc_launch_reduce_mlp(const float* part, NrcControl* ctl, uint32_t capacity, float* w, float* m,
                                  float* v, float* grad_out, NrcHyper hp, bool apply, hipStream_t st);
-// Adam on the grid (or, without `apply`, grid gradient as f32 into
-// grad_out); clears the fixed-point gradients. With `ema` set, also the
-// moving average ema = alpha ema + (1 - alpha) table and its debiased
-// value (step ctl->step + 1) into `inf`.
-hipError_t nrc_launch_adam_grid(float* table, float* m, float* v, unsigned long long* grid_grad,
+// Adam on the grid with the moving average ema = alpha ema + (1 - alpha)
+// table and its debiased value (step ctl->t) into `inf`; without `apply`
+// the grid gradient as f32 into grad_out. Clears the gradients.
+hipError_t nrc_launch_adam_grid(float* table, float* m, float* v, unsigned long long* grid_grad, uint8_t* touched,
                                 uint64_t n, const NrcControl* ctl, float* grad_out, NrcHyper hp, bool apply,
                                 hipStream_t st, float* ema = nullptr, float* inf = nullptr, float alpha = 0.f);
 // The same moving average over the MLP master weights (when ctl->n > 0).

@@ -15,6 +15,8 @@
 // consecutive lanes hit distinct banks).
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 #include "nrc.h"
 
 namespace rrhip {
@@ -120,6 +122,13 @@ __device__ __forceinline__ float2 encode_level(const NrcGridView& G, const float
 // The 24 input values lane half h contributes, in K-slot order: chunks 0
 // and 1 hold the encoding of levels 8c + 2h + {0, 1, 4, 5}, chunk 2 the
 // direction, roughness, albedo (h = 0) or normal and the constant 1 (h = 1).
+// FENCE keeps one level's gathers in flight per lane: without it the
+// scheduler hoists all 64, whose registers cap inference's occupancy;
+// training, with one block of 64 samples on a compute unit, has the
+// registers and waits for one round of gathers instead of eight (a batch of
+// 4,096 samples 29.5 -> 28.2 us; what is left is the chain of six layers
+// there and back).
+template <bool FENCE>
 __device__ __forceinline__ void make_inputs(const NrcGridView& G, const NrcQuery& q, uint32_t h, float v[3][8]) {
   float pn[3];
   normalise(G, q, pn);
@@ -132,9 +141,7 @@ __device__ __forceinline__ void make_inputs(const NrcGridView& G, const NrcQuery
       const float2 f = encode_level(G, pn, lv[i]);
       v[c][2 * i] = f.x;
       v[c][2 * i + 1] = f.y;
-      // Keep one level's gathers in flight per lane: without the fence the
-      // scheduler hoists all 64 and the register count caps occupancy.
-      __builtin_amdgcn_sched_barrier(0);
+      if (FENCE) __builtin_amdgcn_sched_barrier(0);
     }
   }
   if (h == 0) {
@@ -240,7 +247,7 @@ __global__ __launch_bounds__(kInferBlock) void nrc_infer_kernel(NrcGridView G, c
     NrcQuery qq = {};
     if (valid) qq = q[qi];
     float v[3][8];
-    make_inputs(G, qq, h, v);
+    make_inputs<true>(G, qq, h, v);
     bf16x8 in[3];
 #pragma unroll
     for (int c = 0; c < 3; c++) in[c] = pack8(v[c]);
@@ -330,7 +337,7 @@ __device__ __forceinline__ unsigned long long to_fixed(float v) {
 
 __global__ __launch_bounds__(128) void nrc_train_kernel(NrcGridView G, const NrcQuery* __restrict__ q,
                                                        const float* __restrict__ targets,
-                                                       const NrcControl* __restrict__ ctl, float* __restrict__ part,
+                                                       NrcControl* ctl, float* __restrict__ part,
                                                        float* __restrict__ genc) {
   __shared__ __align__(16) uint16_t s_act[6 * kActRows];
   __shared__ __align__(16) uint16_t s_dlt[2 * kActRows];
@@ -338,6 +345,8 @@ __global__ __launch_bounds__(128) void nrc_train_kernel(NrcGridView G, const Nrc
   __shared__ float s_loss[64];
   const uint32_t n = ctl->n;
   const uint32_t base = blockIdx.x * kNrcTrainBlock;
+  // the step's number, for the launches that follow (the last one counts it)
+  if (blockIdx.x == 0 && threadIdx.x == 0) ctl->t = ctl->step + 1;
   if (base >= n) return;  // uniform over the block
   const uint32_t tid = threadIdx.x, lane = tid & 63u, col = lane & 31u, h = lane >> 5, w = tid >> 6;
   const uint32_t sl = 32 * w + col;
@@ -349,7 +358,7 @@ __global__ __launch_bounds__(128) void nrc_train_kernel(NrcGridView G, const Nrc
   NrcQuery qq = {};
   if (valid) qq = q[si];
   float v[3][8];
-  make_inputs(G, qq, h, v);
+  make_inputs<false>(G, qq, h, v);
   bf16x8 a[4];
 #pragma unroll
   for (int c = 0; c < 3; c++) {
@@ -460,11 +469,13 @@ __global__ __launch_bounds__(128) void nrc_train_kernel(NrcGridView G, const Nrc
 // wave's atomic touches the few cache lines of four cells (a corner's two
 // features share a line, and at densely indexed levels so do the +x
 // neighbours) instead of 64 unrelated lines, and the atomics of every
-// sample-level pair are in flight at once.
+// sample-level pair are in flight at once. `touched` marks, per two entries,
+// that a gradient waits there.
 __global__ __launch_bounds__(256) void nrc_grid_scatter_kernel(NrcGridView G, const NrcQuery* __restrict__ q,
                                                               const NrcControl* __restrict__ ctl,
                                                               const float* __restrict__ genc,
-                                                              unsigned long long* __restrict__ gg) {
+                                                              unsigned long long* __restrict__ gg,
+                                                              uint8_t* __restrict__ touched) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t pair = i >> 4, k = i & 15u;
   const uint32_t s = pair / kNrcMaxLevels, l = pair % kNrcMaxLevels;
@@ -479,7 +490,9 @@ __global__ __launch_bounds__(256) void nrc_grid_scatter_kernel(NrcGridView G, co
   const Cell c = cell_of(G, pn, l);
   float wk;
   const uint32_t id = corner(G, l, c, (int)(k >> 1), wk);
-  atomicAdd(gg + (((size_t)l << G.log2_table) + id) * 2 + (k & 1u), to_fixed(gk * wk));
+  const size_t entry = ((size_t)l << G.log2_table) + id;
+  if (!(k & 1u)) touched[entry >> 1] = 1;
+  atomicAdd(gg + entry * 2 + (k & 1u), to_fixed(gk * wk));
 }
 
 __device__ __forceinline__ void adam_update(float& p, float g, float& m, float& v, const NrcHyper& hp, float c1,
@@ -490,7 +503,7 @@ __device__ __forceinline__ void adam_update(float& p, float g, float& m, float& 
 }
 
 __device__ __forceinline__ void bias_corrections(const NrcControl* ctl, const NrcHyper& hp, float& c1, float& c2) {
-  const double t = (double)ctl->step + 1.0;
+  const double t = (double)ctl->t;
   c1 = (float)(1.0 - pow((double)hp.b1, t));
   c2 = (float)(1.0 - pow((double)hp.b2, t));
 }
@@ -501,15 +514,15 @@ __device__ __forceinline__ void bias_corrections(const NrcControl* ctl, const Nr
 constexpr uint32_t kReduceSeg = 8;
 constexpr uint32_t kReduceParams = 256 / kReduceSeg;  // parameters per block
 
-__global__ __launch_bounds__(256) void nrc_reduce_mlp_kernel(const float* __restrict__ part, NrcControl* ctl,
-                                                            float* __restrict__ w, float* __restrict__ m,
-                                                            float* __restrict__ v, float* __restrict__ grad_out,
-                                                            NrcHyper hp, int apply) {
+constexpr uint32_t kReduceBlocks = (kNrcMlpParams + 1 + kReduceParams - 1) / kReduceParams;
+
+// Block `block` of the reduction: returns whether this thread holds the
+// summed gradient s of parameter i (the loss goes into ctl).
+__device__ __forceinline__ bool reduce_mlp(const float* __restrict__ part, NrcControl* ctl, uint32_t block, uint32_t n,
+                                           uint32_t& i, float& s) {
   __shared__ float s_run[kReduceSeg][kReduceParams];
-  const uint32_t n = ctl->n;
-  if (n == 0) return;
   const uint32_t pl = threadIdx.x % kReduceParams, seg = threadIdx.x / kReduceParams;
-  const uint32_t i = blockIdx.x * kReduceParams + pl;
+  i = block * kReduceParams + pl;
   const uint32_t nb = (n + kNrcTrainBlock - 1) / kNrcTrainBlock;
   const uint32_t per = (nb + kReduceSeg - 1) / kReduceSeg;
   float r = 0.f;
@@ -517,37 +530,141 @@ __global__ __launch_bounds__(256) void nrc_reduce_mlp_kernel(const float* __rest
     for (uint32_t b = seg * per; b < min(nb, (seg + 1) * per); b++) r += part[(size_t)b * kNrcPartStride + i];
   s_run[seg][pl] = r;
   __syncthreads();
-  if (seg != 0 || i > kNrcMlpParams) return;
-  float s = 0.f;
+  if (seg != 0 || i > kNrcMlpParams) return false;
+  s = 0.f;
 #pragma unroll
   for (uint32_t k = 0; k < kReduceSeg; k++) s += s_run[k][pl];
   if (i == kNrcMlpParams) {
     ctl->last_loss = s;
-    return;
+    return false;
   }
+  return true;
+}
+
+__device__ __forceinline__ float mlp_adam(float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
+                                          uint32_t i, float g, const NrcHyper& hp, float c1, float c2) {
+  float p = w[i], mm = m[i], vv = v[i];
+  adam_update(p, g, mm, vv, hp, c1, c2);
+  w[i] = p;
+  m[i] = mm;
+  v[i] = vv;
+  return p;
+}
+
+__global__ __launch_bounds__(256) void nrc_reduce_mlp_kernel(const float* __restrict__ part, NrcControl* ctl,
+                                                            float* __restrict__ w, float* __restrict__ m,
+                                                            float* __restrict__ v, float* __restrict__ grad_out,
+                                                            NrcHyper hp, int apply) {
+  const uint32_t n = ctl->n;
+  if (n == 0) return;
+  uint32_t i;
+  float s;
+  if (!reduce_mlp(part, ctl, blockIdx.x, n, i, s)) return;
   if (!apply) {
     grad_out[i] = s;
     return;
   }
   float c1, c2;
   bias_corrections(ctl, hp, c1, c2);
-  float p = w[i], mm = m[i], vv = v[i];
-  adam_update(p, s, mm, vv, hp, c1, c2);
-  w[i] = p;
-  m[i] = mm;
-  v[i] = vv;
+  mlp_adam(w, m, v, i, s, hp, c1, c2);
+}
+
+// Writes parameter i's bf16 copies (the layouts of nrc_pack_kernel; kperm is
+// its own inverse).
+__device__ __forceinline__ void pack_param(uint32_t i, float p, uint16_t* __restrict__ wf, uint16_t* __restrict__ wb) {
+  const uint16_t b = (uint16_t)bf16_bits(p);
+  if (i < kNrcOffW[1]) {
+    const uint32_t r = i / 48, k = i % 48;
+    wf[kNrcFwdOff[0] + r * 48 + kperm(k)] = b;
+    if (k < 32) wb[kNrcBwdOff[0] + k * 64 + kperm(r)] = b;
+  } else if (i < kNrcOffW[5]) {
+    const uint32_t l = 1 + (i - kNrcOffW[1]) / 4096, e = (i - kNrcOffW[1]) % 4096, r = e / 64, k = e % 64;
+    wf[kNrcFwdOff[l] + r * 64 + kperm(k)] = b;
+    wb[kNrcBwdOff[l] + k * 64 + kperm(r)] = b;
+  } else {
+    const uint32_t e = i - kNrcOffW[5], r = e / 64, k = e % 64;
+    wf[kNrcFwdOff[5] + r * 64 + kperm(k)] = b;
+    wb[kNrcBwdOff[5] + k * 16 + kperm(r)] = b;
+  }
+}
+
+// The parameter update of a step without a moving average, in one launch:
+// blocks [0, kReduceBlocks) sum the MLP's partials, step it and write its
+// bf16 copies (and count the step); the others run Adam over the grid, a
+// row of `gx` blocks per level, four parameters a thread with 16-byte
+// accesses (the tables are 256-byte aligned).
+//
+// Adam moves every parameter that has ever had a gradient in every step, so
+// the pass is bound by moving it and its two moments, 24 B each. It leaves
+// out what cannot change anything: gradients (8 B) are read, and cleared,
+// only where `touched` says one waits, and a densely indexed level stops at
+// its last grid corner, `used` entries (what lies behind it is never
+// looked up; its moments stay zero, and a step by zero changes nothing as
+// long as epsilon > 0 and the rate is finite). 16 levels of 2^19 entries,
+// 12.2 million parameters in use: 60 us (4.9 TB/s, a large copy's rate) in
+// place of 108 us for the reduction, an Adam pass that read every gradient
+// and a packing launch; 64 steps of 4,096 samples with the read-back of the
+// parameters 21.5 -> 17.4 ms, although marking costs the scatter pass 2 of
+// 19 us.
+struct GridUse {
+  uint32_t groups[kNrcMaxLevels];  // 4-parameter groups in use per level
+};
+__global__ __launch_bounds__(256) void nrc_update_kernel(const float* __restrict__ part, NrcControl* ctl,
+                                                        float* __restrict__ w, float* __restrict__ wm,
+                                                        float* __restrict__ wv, uint16_t* __restrict__ wf,
+                                                        uint16_t* __restrict__ wb, float4* __restrict__ table,
+                                                        float4* __restrict__ m, float4* __restrict__ v,
+                                                        ulonglong2* __restrict__ gg, uint8_t* __restrict__ touched,
+                                                        GridUse use, uint32_t log2_groups, uint32_t gx, NrcHyper hp) {
+  const uint32_t n = ctl->n;
+  if (n == 0) return;
+  float c1, c2;
+  bias_corrections(ctl, hp, c1, c2);
+  if (blockIdx.x < kReduceBlocks) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl->step = ctl->t;
+    uint32_t i;
+    float s;
+    if (reduce_mlp(part, ctl, blockIdx.x, n, i, s)) pack_param(i, mlp_adam(w, wm, wv, i, s, hp, c1, c2), wf, wb);
+    return;
+  }
+  const uint32_t b = blockIdx.x - kReduceBlocks, l = b / gx;
+  for (uint32_t k = (b % gx) * blockDim.x + threadIdx.x; k < use.groups[l]; k += gx * blockDim.x) {
+    const size_t j = ((size_t)l << log2_groups) + k;
+    long long fx[4] = {0, 0, 0, 0};
+    if (touched[j]) {
+      const ulonglong2 ga = gg[2 * j], gb = gg[2 * j + 1];
+      fx[0] = (long long)ga.x;
+      fx[1] = (long long)ga.y;
+      fx[2] = (long long)gb.x;
+      fx[3] = (long long)gb.y;
+      gg[2 * j] = make_ulonglong2(0ull, 0ull);
+      gg[2 * j + 1] = make_ulonglong2(0ull, 0ull);
+      touched[j] = 0;
+    }
+    float4 p = table[j], mm = m[j], vv = v[j];
+    adam_update(p.x, (float)fx[0] * (1.f / 68719476736.f), mm.x, vv.x, hp, c1, c2);
+    adam_update(p.y, (float)fx[1] * (1.f / 68719476736.f), mm.y, vv.y, hp, c1, c2);
+    adam_update(p.z, (float)fx[2] * (1.f / 68719476736.f), mm.z, vv.z, hp, c1, c2);
+    adam_update(p.w, (float)fx[3] * (1.f / 68719476736.f), mm.w, vv.w, hp, c1, c2);
+    table[j] = p;
+    m[j] = mm;
+    v[j] = vv;
+  }
 }
 
 // Moving average of the parameters for inference: e_t = a e_{t-1} +
 // (1 - a) p_t, used as e_t / (1 - a^t) (t counts steps since the
 // parameters were set).
 __device__ __forceinline__ float ema_debias(const NrcControl* ctl, float a) {
-  return (float)(1.0 / (1.0 - pow((double)a, (double)ctl->step + 1.0)));
+  return (float)(1.0 / (1.0 - pow((double)a, (double)ctl->t)));
 }
 
+// The grid's update with a moving average for inference (apply), or its
+// gradient alone; clears the gradients.
 __global__ __launch_bounds__(256) void nrc_adam_grid_kernel(float* __restrict__ table, float* __restrict__ m,
                                                            float* __restrict__ v, unsigned long long* __restrict__ gg,
-                                                           uint64_t n, const NrcControl* __restrict__ ctl,
+                                                           uint8_t* __restrict__ touched, uint64_t n,
+                                                           const NrcControl* __restrict__ ctl,
                                                            float* __restrict__ grad_out, NrcHyper hp, int apply,
                                                            float* __restrict__ ema, float* __restrict__ inf,
                                                            float alpha) {
@@ -556,56 +673,23 @@ __global__ __launch_bounds__(256) void nrc_adam_grid_kernel(float* __restrict__ 
   if (apply) bias_corrections(ctl, hp, c1, c2);
   const float corr = ema ? ema_debias(ctl, alpha) : 1.f;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  const uint64_t t0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const auto one = [&](uint64_t i, long long fx) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const long long fx = (long long)gg[i];
+    if (fx != 0) gg[i] = 0ull;
+    if ((i & 3u) == 0) touched[i >> 2] = 0;
     const float g = (float)fx * (1.f / 68719476736.f);
     if (!apply) {
       grad_out[i] = g;
-      return;
+      continue;
     }
     float p = table[i], mm = m[i], vv = v[i];
     adam_update(p, g, mm, vv, hp, c1, c2);
     table[i] = p;
     m[i] = mm;
     v[i] = vv;
-    if (ema) {
-      const float e = alpha * ema[i] + (1.f - alpha) * p;
-      ema[i] = e;
-      inf[i] = e * corr;
-    }
-  };
-  if (apply && !ema) {
-    // four parameters per thread with 16-byte accesses (the tables are
-    // 256-byte aligned); the gradients are cleared where any was set
-    const uint64_t n4 = n / 4;
-    for (uint64_t j = t0; j < n4; j += stride) {
-      ulonglong2* g2 = (ulonglong2*)gg + 2 * j;
-      const ulonglong2 ga = g2[0], gb = g2[1];
-      const long long fx[4] = {(long long)ga.x, (long long)ga.y, (long long)gb.x, (long long)gb.y};
-      if (fx[0] | fx[1] | fx[2] | fx[3]) {
-        g2[0] = make_ulonglong2(0ull, 0ull);
-        g2[1] = make_ulonglong2(0ull, 0ull);
-      }
-      float4 p = ((float4*)table)[j], mm = ((float4*)m)[j], vv = ((float4*)v)[j];
-      adam_update(p.x, (float)fx[0] * (1.f / 68719476736.f), mm.x, vv.x, hp, c1, c2);
-      adam_update(p.y, (float)fx[1] * (1.f / 68719476736.f), mm.y, vv.y, hp, c1, c2);
-      adam_update(p.z, (float)fx[2] * (1.f / 68719476736.f), mm.z, vv.z, hp, c1, c2);
-      adam_update(p.w, (float)fx[3] * (1.f / 68719476736.f), mm.w, vv.w, hp, c1, c2);
-      ((float4*)table)[j] = p;
-      ((float4*)m)[j] = mm;
-      ((float4*)v)[j] = vv;
-    }
-    for (uint64_t i = 4 * n4 + t0; i < n; i += stride) {
-      const long long fx = (long long)gg[i];
-      if (fx != 0) gg[i] = 0ull;
-      one(i, fx);
-    }
-    return;
-  }
-  for (uint64_t i = t0; i < n; i += stride) {
-    const long long fx = (long long)gg[i];
-    if (fx != 0) gg[i] = 0ull;
-    one(i, fx);
+    const float e = alpha * ema[i] + (1.f - alpha) * p;
+    ema[i] = e;
+    inf[i] = e * corr;
   }
 }
 
@@ -623,7 +707,7 @@ __global__ __launch_bounds__(256) void nrc_ema_mlp_kernel(const float* __restric
 __global__ __launch_bounds__(256) void nrc_pack_kernel(const float* __restrict__ w, uint16_t* __restrict__ wf,
                                                       uint16_t* __restrict__ wb, NrcControl* ctl, int count_step) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0 && count_step && ctl->n > 0) ctl->step += 1;
+  if (i == 0 && count_step && ctl->n > 0) ctl->step = ctl->t;
   if (i < kNrcFwdSize) {
     float val;
     if (i < kNrcFwdOff[1]) {
@@ -678,33 +762,52 @@ hipError_t nrc_launch_infer_paths(const NrcGridView& G, const NrcQuery* q, const
   return hipGetLastError();
 }
 
-hipError_t nrc_launch_train(const NrcGridView& G, const NrcQuery* q, const float* targets, const NrcControl* ctl,
+hipError_t nrc_launch_train(const NrcGridView& G, const NrcQuery* q, const float* targets, NrcControl* ctl,
                             uint32_t capacity, float* part, float* genc, unsigned long long* grid_grad,
-                            hipStream_t st) {
+                            uint8_t* touched, hipStream_t st) {
   const uint32_t blocks = (capacity + kNrcTrainBlock - 1) / kNrcTrainBlock;
   hipLaunchKernelGGL(nrc_train_kernel, dim3(blocks < 1 ? 1 : blocks), dim3(128), 0, st, G, q, targets, ctl, part,
                      genc);
   const uint64_t lanes = (uint64_t)(capacity < 1 ? 1 : capacity) * kNrcMaxLevels * 16;
   hipLaunchKernelGGL(nrc_grid_scatter_kernel, dim3((uint32_t)((lanes + 255) / 256)), dim3(256), 0, st, G, q, ctl,
-                     genc, grid_grad);
+                     genc, grid_grad, touched);
   return hipGetLastError();
 }
 
 hipError_t nrc_launch_reduce_mlp(const float* part, NrcControl* ctl, uint32_t capacity, float* w, float* m, float* v,
                                  float* grad_out, NrcHyper hp, bool apply, hipStream_t st) {
   (void)capacity;
-  hipLaunchKernelGGL(nrc_reduce_mlp_kernel, dim3((kNrcMlpParams + 1 + kReduceParams - 1) / kReduceParams), dim3(256),
-                     0, st, part, ctl, w, m, v, grad_out, hp, apply ? 1 : 0);
+  hipLaunchKernelGGL(nrc_reduce_mlp_kernel, dim3(kReduceBlocks), dim3(256), 0, st, part, ctl, w, m, v, grad_out, hp,
+                     apply ? 1 : 0);
   return hipGetLastError();
 }
 
-hipError_t nrc_launch_adam_grid(float* table, float* m, float* v, unsigned long long* grid_grad, uint64_t n,
-                                const NrcControl* ctl, float* grad_out, NrcHyper hp, bool apply, hipStream_t st,
-                                float* ema, float* inf, float alpha) {
+hipError_t nrc_launch_update(const NrcGridView& G, const float* part, NrcControl* ctl, float* w, float* wm, float* wv,
+                             uint16_t* wf, uint16_t* wb, float* table, float* m, float* v,
+                             unsigned long long* grid_grad, uint8_t* touched, NrcHyper hp, hipStream_t st) {
+  GridUse use{};
+  uint32_t most = 0;
+  for (uint32_t l = 0; l < G.levels; l++) {
+    uint64_t entries = 1ull << G.log2_table;
+    const uint64_t n1 = (uint64_t)G.res[l] + 1;
+    if (((G.dense_mask >> l) & 1u) && hp.eps > 0.f && std::isfinite(hp.lr)) entries = n1 * n1 * n1;
+    use.groups[l] = (uint32_t)((entries + 1) / 2);
+    most = use.groups[l] > most ? use.groups[l] : most;
+  }
+  const uint32_t gx = (most + 511) / 512;  // two groups per thread of the fullest level
+  hipLaunchKernelGGL(nrc_update_kernel, dim3(kReduceBlocks + gx * G.levels), dim3(256), 0, st, part, ctl, w, wm, wv, wf,
+                     wb, (float4*)table, (float4*)m, (float4*)v, (ulonglong2*)grid_grad, touched, use,
+                     G.log2_table - 1, gx, hp);
+  return hipGetLastError();
+}
+
+hipError_t nrc_launch_adam_grid(float* table, float* m, float* v, unsigned long long* grid_grad, uint8_t* touched,
+                                uint64_t n, const NrcControl* ctl, float* grad_out, NrcHyper hp, bool apply,
+                                hipStream_t st, float* ema, float* inf, float alpha) {
   const uint64_t b = (n + 255) / 256;
   const uint32_t blocks = (uint32_t)(b > 8192 ? 8192 : (b < 1 ? 1 : b));
-  hipLaunchKernelGGL(nrc_adam_grid_kernel, dim3(blocks), dim3(256), 0, st, table, m, v, grid_grad, n, ctl, grad_out,
-                     hp, apply ? 1 : 0, ema, inf, alpha);
+  hipLaunchKernelGGL(nrc_adam_grid_kernel, dim3(blocks), dim3(256), 0, st, table, m, v, grid_grad, touched, n, ctl,
+                     grad_out, hp, apply ? 1 : 0, ema, inf, alpha);
   return hipGetLastError();
 }
 

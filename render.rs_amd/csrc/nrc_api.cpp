@@ -137,16 +137,20 @@ void nrc_set_bounds(rrhip_nrc* c, const float lo[3], const float hi[3]) {
 
 hipError_t nrc_step_device(rrhip_nrc* c, const NrcQuery* q, const float* targets, uint32_t capacity,
                            hipStream_t st) {
-  hipError_t e = nrc_launch_train(c->G, q, targets, c->d_ctl, capacity, c->d_part, c->d_genc, c->d_tg, st);
+  hipError_t e = nrc_launch_train(c->G, q, targets, c->d_ctl, capacity, c->d_part, c->d_genc, c->d_tg, c->d_touched, st);
+  if (!c->d_inf_table) {
+    if (e == hipSuccess)
+      e = nrc_launch_update(c->G, c->d_part, c->d_ctl, c->d_w, c->d_wm, c->d_wv, c->d_wf, c->d_wb, c->d_table, c->d_tm,
+                            c->d_tv, c->d_tg, c->d_touched, c->hp, st);
+    return e;
+  }
   if (e == hipSuccess)
     e = nrc_launch_reduce_mlp(c->d_part, c->d_ctl, capacity, c->d_w, c->d_wm, c->d_wv, nullptr, c->hp, true, st);
   if (e == hipSuccess)
-    e = nrc_launch_adam_grid(c->d_table, c->d_tm, c->d_tv, c->d_tg, c->grid_n, c->d_ctl, nullptr, c->hp, true, st,
-                             c->d_ema_table, c->d_inf_table, c->cfg.ema);
-  if (e == hipSuccess && c->d_inf_table) {
-    e = nrc_launch_ema_mlp(c->d_w, c->d_ema_w, c->d_inf_w, c->d_ctl, c->cfg.ema, st);
-    if (e == hipSuccess) e = nrc_launch_pack(c->d_inf_w, c->d_inf_wf, nullptr, c->d_ctl, false, st);
-  }
+    e = nrc_launch_adam_grid(c->d_table, c->d_tm, c->d_tv, c->d_tg, c->d_touched, c->grid_n, c->d_ctl, nullptr, c->hp,
+                             true, st, c->d_ema_table, c->d_inf_table, c->cfg.ema);
+  if (e == hipSuccess) e = nrc_launch_ema_mlp(c->d_w, c->d_ema_w, c->d_inf_w, c->d_ctl, c->cfg.ema, st);
+  if (e == hipSuccess) e = nrc_launch_pack(c->d_inf_w, c->d_inf_wf, nullptr, c->d_ctl, false, st);
   if (e == hipSuccess) e = nrc_launch_pack(c->d_w, c->d_wf, c->d_wb, c->d_ctl, true, st);
   return e;
 }
@@ -190,6 +194,7 @@ int rrhip_nrc_create(rrhip_ctx* ctx, const rrhip_nrc_config* config, rrhip_nrc**
   if (e == hipSuccess) e = alloc_n(c, &c->d_tm, c->grid_n);
   if (e == hipSuccess) e = alloc_n(c, &c->d_tv, c->grid_n);
   if (e == hipSuccess) e = alloc_n(c, &c->d_tg, c->grid_n);
+  if (e == hipSuccess) e = alloc_n(c, &c->d_touched, c->grid_n / 4);
   if (e == hipSuccess) e = alloc_n(c, &c->d_w, (uint64_t)kNrcMlpParams);
   if (e == hipSuccess) e = alloc_n(c, &c->d_wm, (uint64_t)kNrcMlpParams);
   if (e == hipSuccess) e = alloc_n(c, &c->d_wv, (uint64_t)kNrcMlpParams);
@@ -290,6 +295,7 @@ int rrhip_nrc_set_params(rrhip_nrc* c, const float* mlp, const float* grid) {
   RRHIP_HIP_TRY(hipMemsetAsync(c->d_tm, 0, c->grid_n * sizeof(float), st));
   RRHIP_HIP_TRY(hipMemsetAsync(c->d_tv, 0, c->grid_n * sizeof(float), st));
   RRHIP_HIP_TRY(hipMemsetAsync(c->d_tg, 0, c->grid_n * sizeof(unsigned long long), st));
+  RRHIP_HIP_TRY(hipMemsetAsync(c->d_touched, 0, c->grid_n / 4, st));
   RRHIP_HIP_TRY(hipMemsetAsync(c->d_ctl, 0, sizeof(NrcControl), st));
   RRHIP_HIP_TRY(nrc_launch_pack(c->d_w, c->d_wf, c->d_wb, c->d_ctl, false, st));
   if (c->d_inf_table) {  // averages restart from the parameters set
@@ -366,11 +372,12 @@ int rrhip_nrc_gradients(rrhip_nrc* c, const rrhip_nrc_query* queries, const floa
   if (int s = stage_batch(c, queries, targets, n, "rrhip_nrc_gradients")) return s;
   hipStream_t st = c->ctx->stream;
   if (!c->d_gout) RRHIP_HIP_TRY(alloc_n(c, &c->d_gout, c->grid_n));
-  RRHIP_HIP_TRY(nrc_launch_train(c->G, c->d_q, c->d_t, c->d_ctl, (uint32_t)n, c->d_part, c->d_genc, c->d_tg, st));
+  RRHIP_HIP_TRY(nrc_launch_train(c->G, c->d_q, c->d_t, c->d_ctl, (uint32_t)n, c->d_part, c->d_genc, c->d_tg,
+                                 c->d_touched, st));
   RRHIP_HIP_TRY(nrc_launch_reduce_mlp(c->d_part, c->d_ctl, (uint32_t)n, c->d_w, c->d_wm, c->d_wv, c->d_wgrad, c->hp,
                                       false, st));
-  RRHIP_HIP_TRY(nrc_launch_adam_grid(c->d_table, c->d_tm, c->d_tv, c->d_tg, c->grid_n, c->d_ctl, c->d_gout, c->hp,
-                                     false, st));
+  RRHIP_HIP_TRY(nrc_launch_adam_grid(c->d_table, c->d_tm, c->d_tv, c->d_tg, c->d_touched, c->grid_n, c->d_ctl,
+                                     c->d_gout, c->hp, false, st));
   if (mlp_grad)
     RRHIP_HIP_TRY(hipMemcpyAsync(mlp_grad, c->d_wgrad, kNrcMlpParams * sizeof(float), hipMemcpyDeviceToHost, st));
   if (grid_grad)

@@ -18,6 +18,7 @@ struct rrhip_nrc {
   float* d_tm = nullptr;
   float* d_tv = nullptr;
   unsigned long long* d_tg = nullptr;
+  uint8_t* d_touched = nullptr;  // per 4 grid parameters: a gradient waits in d_tg
   float* d_w = nullptr;
   float* d_wm = nullptr;
   float* d_wv = nullptr;
