@@ -39,7 +39,7 @@ hipError_t pt_launch_set_u64(uint64_t* dst, uint64_t v, hipStream_t st);
 // paths terminate into radiance-cache queries (see NrcPathBuffers).
 // ev (profiling, may be null): four events recorded before extend, before
 // shade (the queue sort included), before shadow, and after it.
-hipError_t pt_launch_bounce(const PtSceneView& S, const PathBuffers& P, const PtParams& prm,
+hipError_t pt_launch_bounce(const PtSceneView& S, PathBuffers P, const PtParams& prm,
                             const uint32_t* q, uint32_t* qnext, uint32_t capacity, const NrcPathBuffers& N,
                             hipStream_t st, const hipEvent_t* ev = nullptr);
 // The shadow rays of the last round (P.round = the number of rounds).
@@ -51,6 +51,13 @@ hipError_t pt_launch_last_shadows(const PtSceneView& S, const PathBuffers& P, ui
 enum TraceWork { kTraceExtend, kTraceShadow, kTraceRound };
 hipError_t pt_launch_trace(const PtSceneView& S, const PathBuffers& P, const uint32_t* q, uint32_t gt, TraceWork work,
                            hipStream_t st);
+// How many paths at most a tail launch of round P.round finishes by itself
+// (0: no tail launch in this round; ~0u: any number, the pass ends there).
+uint32_t pt_tail_limit(const PtSceneView& S, const PathBuffers& P, const NrcPathBuffers& N);
+// The tail launch: the live paths of the round, from their closest hits to
+// their ends, if they are at most `limit`.
+hipError_t pt_launch_tail(const PtSceneView& S, const PathBuffers& P, const PtParams& prm, const uint32_t* q,
+                          const NrcPathBuffers& N, uint32_t limit, hipStream_t st);
 // The shading kernel of one bounce over the queue `qshade`, with
 // error-bounded ray origins or render.rs's fixed push (S.ray_offset > 0).
 hipError_t pt_launch_shade_bounded(const PtSceneView& S, const PathBuffers& P, const PtParams& prm,

@@ -384,7 +384,7 @@ static uint32_t trace_grid(uint64_t capacity) {
   return (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(1, b));
 }
 
-hipError_t pt_launch_bounce(const PtSceneView& S, const PathBuffers& P, const PtParams& prm, const uint32_t* q,
+hipError_t pt_launch_bounce(const PtSceneView& S, PathBuffers P, const PtParams& prm, const uint32_t* q,
                             uint32_t* qnext, uint32_t capacity, const NrcPathBuffers& N, hipStream_t st,
                             const hipEvent_t* ev) {
   const uint32_t g = grid_for(capacity);
@@ -394,6 +394,11 @@ hipError_t pt_launch_bounce(const PtSceneView& S, const PathBuffers& P, const Pt
   hipError_t e = pt_launch_trace(S, P, q, gt, merged ? kTraceRound : kTraceExtend, st);
   if (e != hipSuccess) return e;
   if (ev) (void)hipEventRecord(ev[1], st);
+  P.taken = pt_tail_limit(S, P, N);
+  if (P.taken) {
+    e = pt_launch_tail(S, P, prm, q, N, P.taken, st);
+    if (e != hipSuccess || P.taken == 0xFFFFFFFFu) return e;
+  }
   const uint32_t* qshade = q;
   if (P.qs) {  // group the queue by shading class so shade waves run one BSDF kind
     hipLaunchKernelGGL(sort_count_kernel, dim3(kSortBlocks), dim3(kBlock), 0, st, S, P, q);

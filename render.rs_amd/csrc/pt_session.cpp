@@ -276,13 +276,16 @@ hipError_t enqueue_pass(rrhip_session* s, uint32_t n, uint32_t ncol, const uint3
     ev = s->prof_ev.data();
   }
   if (e == hipSuccess) e = pt_launch_raygen(s->S, P, prm, total, N, sample0_dev, st);
+  uint32_t done = 0;
   for (uint32_t b = 0; b < rounds && e == hipSuccess; b++) {
     const uint32_t* q = (b & 1) ? P.q1 : P.q0;
     uint32_t* qn = (b & 1) ? P.q0 : P.q1;
     P.round = b;
     e = pt_launch_bounce(s->S, P, prm, q, qn, paths, N, st, prof ? ev + 4 * b : nullptr);
+    done = b + 1;
+    if (pt_tail_limit(s->S, P, N) == 0xFFFFFFFFu) break;
   }
-  P.round = rounds;
+  P.round = done;
   if (e == hipSuccess) e = pt_launch_last_shadows(s->S, P, paths, st);
   hipEvent_t* ev_nrc = prof ? ev + 4 * rounds : nullptr;
   bool nrc_timed = false, steps_timed = false;

@@ -350,6 +350,7 @@ struct PathBuffers {
   // raygen, so no launch is needed between rounds.
   unsigned long long* rounds;
   uint32_t round;   // the round a launch works on (set by the host for each launch)
+  uint32_t taken;   // the round's paths were finished by a tail launch if they are at most this many
   __device__ uint32_t live() const { return (uint32_t)rounds[round]; }
   __device__ uint32_t shadows() const { return (uint32_t)(rounds[round] >> 32); }
   __device__ unsigned long long* append() const { return rounds + round + 1; }

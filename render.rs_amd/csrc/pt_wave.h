@@ -844,7 +844,7 @@ template <bool NRC, bool TR, bool MEDIA, bool FILM, bool FIXED, bool HAIR, bool 
 __device__ __forceinline__ void shade_pass(const PtSceneView& S, const PathBuffers& P, const PtParams& prm,
                                            const uint32_t* __restrict__ q, uint32_t* __restrict__ qnext,
                                            const NrcPathBuffers& N) {
-  const uint32_t n = P.live();
+  const uint32_t live = P.live(), n = live <= P.taken ? 0 : live;
   const uint32_t stride = gridDim.x * blockDim.x;
   // Block-uniform loop bound so every lane reaches the append.
   for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
