@@ -36,6 +36,7 @@ struct rrhip_batch {
   uint32_t* d_next = nullptr;
   uint32_t* d_left = nullptr;
   unsigned long long* d_clock = nullptr;
+  float4* d_samples = nullptr;  // the waves' samples that wait for their chunk's end
 };
 
 namespace {
@@ -336,6 +337,7 @@ hipError_t persistent_setup(rrhip_batch* b) {
   if (e == hipSuccess) e = alloc_n(b, &b->d_next, 1);
   if (e == hipSuccess) e = alloc_n(b, &b->d_left, nj);
   if (e == hipSuccess) e = alloc_n(b, &b->d_clock, (uint64_t)nj + 1);
+  if (e == hipSuccess) e = alloc_n(b, &b->d_samples, n * kPtChunkSamples);
   if (e == hipSuccess) e = alloc_n(b, &b->d_pjobs, nj);
   return e;
 }
@@ -353,7 +355,8 @@ int rrhip_batch_render_persistent(rrhip_batch* b, double* job_ms, double* total_
   hipStream_t st = b->ctx->stream;
   RRHIP_HIP_TRY(persistent_setup(b));
   const uint32_t nj = (uint32_t)b->jobs.size();
-  // items: every pixel of every job, jobs shortest first (samples x pixels)
+  // items: chunks of whole pixels, at most kPtChunkSamples samples each
+  // (four pixels where one has more), jobs shortest first (samples x pixels)
   std::vector<uint32_t> order(nj);
   for (uint32_t j = 0; j < nj; j++) order[j] = j;
   std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) {
@@ -361,7 +364,7 @@ int rrhip_batch_render_persistent(rrhip_batch* b, double* job_ms, double* total_
   });
   std::vector<PtJob> table(nj);
   std::vector<uint32_t> left(nj), pos(nj);
-  uint64_t items = 0;
+  uint64_t items = 0, pixels = 0;
   for (uint32_t k = 0; k < nj; k++) {
     const uint32_t j = order[k];
     const rrhip_batch_job& J = b->jobs[j];
@@ -375,12 +378,14 @@ int rrhip_batch_render_persistent(rrhip_batch* b, double* job_ms, double* total_
     t.prm.spp_pass = J.spp;
     t.prm.sample0 = J.params.sample_base;
     t.pix_begin = (uint32_t)items;
+    t.chunk_pix = J.spp > kPtChunkSamples ? 4u : kPtChunkSamples / J.spp;
     t.accum = b->accum[j];
     left[k] = b->npix[j];
     pos[j] = k;
-    items += b->npix[j];
+    items += (b->npix[j] + t.chunk_pix - 1) / t.chunk_pix;
+    pixels += b->npix[j];
   }
-  if (items >= (1ull << 32)) return fail(RRHIP_ERR_INVALID_ARGUMENT, "rrhip_batch_render_persistent: too many pixels");
+  if (pixels >= (1ull << 32)) return fail(RRHIP_ERR_INVALID_ARGUMENT, "rrhip_batch_render_persistent: too many pixels");
   for (uint32_t j = 0; j < nj; j++)
     RRHIP_HIP_TRY(hipMemsetAsync(b->accum[j], 0, (size_t)b->npix[j] * RRHIP_ACCUM_STRIDE * sizeof(double), st));
   const std::vector<unsigned long long> clock0(nj + 1, ~0ull);
@@ -393,7 +398,7 @@ int rrhip_batch_render_persistent(rrhip_batch* b, double* job_ms, double* total_
   RRHIP_HIP_TRY(hipMemcpyAsync(b->d_next, &zero, sizeof(zero), hipMemcpyHostToDevice, st));
   RRHIP_HIP_TRY(hipEventRecord(b->ctx->ev0, st));
   RRHIP_HIP_TRY(pt_launch_batch_persistent(b->d_pjobs, nj, b->PP, (uint32_t)items, b->p_lanes, b->p_flags, b->d_next,
-                                           b->d_left, b->d_clock, st));
+                                           b->d_left, b->d_clock, b->d_samples, st));
   RRHIP_HIP_TRY(hipEventRecord(b->ctx->ev1, st));
   RRHIP_HIP_TRY(hipEventSynchronize(b->ctx->ev1));
   float ms = 0.f;

@@ -414,8 +414,12 @@ struct PtParams {
 struct PtJob {
   PtSceneView S;
   PtParams prm;
-  uint32_t slot_begin, pix_begin;
+  uint32_t slot_begin, pix_begin;  // persistent launch: pix_begin counts chunks of chunk_pix pixels
+  uint32_t chunk_pix;
   double* accum;
 };
+
+// The persistent launch: samples of one chunk of work at most.
+constexpr uint32_t kPtChunkSamples = 64;
 
 }  // namespace rrhip
