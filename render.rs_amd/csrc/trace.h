@@ -46,8 +46,9 @@ enum class TraceMode : int;
 // Wave slots of the current device that hold the query kernel of this
 // tuning and mode at once (0 if unknown).
 uint64_t trace_resident_waves(const TraceTuning& tu, TraceMode mode);
-// Rays per wave that spread `n` rays over `slots` resident waves (whole
-// wavefronts of rays, at least 64, at most 2^20; 256 when slots is 0).
+// Rays per wave that spread `n` rays over `slots` resident waves: whole
+// wavefronts of rays, at most 2^20, or 4, 8, 16 or 32 where n is too small
+// to fill the device; 256 when slots is 0.
 uint32_t fill_chunk(uint64_t n, uint64_t slots);
 
 // Smallest supported stack size holding `depth` entries (0 if none does).

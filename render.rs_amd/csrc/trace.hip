@@ -18,7 +18,7 @@
 // Execution (wave64): every wave owns a contiguous chunk of rays, by
 // default sized so that the launch's waves all fit the device at once
 // (one round, no tail of late waves; a shared atomic ray counter measured
-// slower). The kernel is bound by vector-instruction issue, and per-ray work varies by
+// slower), with fewer than 64 lanes at work where the batch is small. The kernel is bound by vector-instruction issue, and per-ray work varies by
 // an order of magnitude between rays, so the wave schedules phases rather
 // than letting lanes wait on each other's loops: each iteration, three
 // ballots count the lanes that walk interior nodes, the lanes that hold a
@@ -209,8 +209,20 @@ uint64_t trace_resident_waves(const TraceTuning& tu, TraceMode mode) {
   return any ? slots_block<true, 2>(tu) : slots_block<false, 2>(tu);
 }
 
+// Batches too small to fill the device run with fewer lanes per wave: such a
+// launch lasts as long as its slowest wave, whose lanes' steps wait for each
+// other, while issue slots are free. Four lanes at least (two were slower at
+// 3,000 rays already), and more as soon as half of the wave slots would
+// start, since more waves than that share the vector units. Closest hits
+// from device memory against 160,000 triangles, launch and
+// synchronisation included, with 64 lanes and with the rule's 4 / 8 / 16 /
+// 32: 8,000 rays 101 -> 85 us, 20,000 117 -> 105, 40,000 117 -> 108, 80,000
+// 127 -> 115; at 140,000 32 lanes lose (154 -> 160), at 340,000 48 (171 ->
+// 208). Any hits alike (8,000: 99 -> 82).
 uint32_t fill_chunk(uint64_t n, uint64_t slots) {
   if (slots == 0) return 256;
+  for (uint32_t lanes = 4; lanes < 64; lanes *= 2)
+    if (n <= slots / 2 * lanes) return lanes;
   const uint64_t per = (n + slots - 1) / slots;
   return (uint32_t)std::min<uint64_t>(std::max<uint64_t>((per + 63) / 64 * 64, 64), 1u << 20);
 }
