@@ -388,7 +388,9 @@ hipError_t pt_launch_bounce(const PtSceneView& S, PathBuffers P, const PtParams&
                             uint32_t* qnext, uint32_t capacity, const NrcPathBuffers& N, hipStream_t st,
                             const hipEvent_t* ev) {
   const uint32_t g = grid_for(capacity);
-  const uint32_t gt = trace_grid(capacity);
+  // the counting kernels end with a few same-address atomics per wave, so
+  // they keep to fewer, striding waves
+  const uint32_t gt = P.prof ? grid_for(capacity, kTraceBlock) : trace_grid(capacity);
   const bool merged = !P.prof && !S.transparent;
   if (ev) (void)hipEventRecord(ev[0], st);
   hipError_t e = pt_launch_trace(S, P, q, gt, merged ? kTraceRound : kTraceExtend, st);

