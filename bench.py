@@ -89,8 +89,9 @@ def cpu_baseline(pos, idx, rays):
 # (the B model): the ray's path state and the record it writes, plus what
 # its traversal fetches as the profiling kernels count it — 64-byte nodes,
 # 48-byte triangle records, 80 bytes per instance entered (instance and
-# mesh records) — and every loose object (64-byte triangles, 32-byte
-# spheres, 128-byte quadrics), which each ray tests.
+# mesh records). The loose objects, which every ray tests, are a few KB that
+# the nearest caches hold and count nothing: with them a box room's 22
+# would move 18.8 TB/s.
 EXTEND_STATE_BYTES = 4 + 32 + 52   # queue entry; origin, direction; hit normal/t, material, two origins
 SHADOW_STATE_BYTES = 4 + 48 + 32   # queue entry; origin, direction, contribution; radiance read + write
 HBM_PEAK = 8000.0  # GB/s
@@ -100,14 +101,12 @@ NRC_TRAIN_FLOP = 3 * NRC_FWD_FLOP                   # forward, input gradients, 
 NRC_QUERY_BYTES = 64 + 16 * 8 * 8 + 16 + 32          # record; 16 levels x 8 corners x 2 f32; throughput; radiance
 
 
-def trace_roofline(prof, scene):
+def trace_roofline(prof):
     """B-model roofline of the extend and shadow kernels from a profile
-    (rrhip_session_get_profile) of the scene description."""
-    loose = 64 * scene.num_triangles + 32 * scene.num_spheres + 128 * scene.num_quadrics
-
+    (rrhip_session_get_profile)."""
     def model(kind, state):
         rays = prof[f"{kind}_rays"]
-        b = (state + loose) * rays + 64 * prof[f"{kind}_nodes"] + 48 * prof[f"{kind}_triangles"] + \
+        b = state * rays + 64 * prof[f"{kind}_nodes"] + 48 * prof[f"{kind}_triangles"] + \
             80 * prof[f"{kind}_instances"]
         ms = prof[f"{kind}_ms"]
         return {"rays": int(rays), "bytes_per_ray": round(b / max(rays, 1), 1),
@@ -123,8 +122,8 @@ def trace_roofline(prof, scene):
             "frac": round(achieved / HBM_PEAK, 4), "traffic": None,
             "kernels": {"extend": ext, "shadow": sh, "shade_ms": round(prof["shade_ms"], 3)},
             "note": "extend + shadow kernels over one profiled frame: B-model bytes (path state, node / "
-                    "triangle / instance fetches counted by the profiling kernels, loose objects) over "
-                    "their event-timed device time"}
+                    "triangle / instance fetches counted by the profiling kernels) over their event-timed "
+                    "device time"}
 
 
 def profiled_frame(ps, params, start, count, nrc_config=None, ctx=None):
@@ -173,7 +172,7 @@ def box_room(ctx, args, with_cpu):
         "rays_per_frame": int(rays),
     }
     se.close()
-    out["roofline"] = trace_roofline(profiled_frame(ps, p, 0, 16), d)
+    out["roofline"] = trace_roofline(profiled_frame(ps, p, 0, 16))
     ps.close()
     if with_cpu:
         sys.path.insert(0, os.path.join(ROOT, "oracle"))
@@ -224,7 +223,7 @@ def instanced_pt(ctx, args, with_cpu):
         "rays_per_frame": int(rays),
         "samples_per_s": round(W * H * SPP / dt, 1),
         "launch_mode": mode,
-        "roofline": trace_roofline(profiled_frame(ps, p, 0, 8), d),
+        "roofline": trace_roofline(profiled_frame(ps, p, 0, 8)),
     }
     if with_cpu:
         # the oracle's plain path tracer on the same scene at 480x270 and
@@ -285,7 +284,7 @@ def hair_curves(ctx, args, with_cpu):
         "mrays_per_s": round(rays / dt / 1e6, 1),
         "rays_per_frame": int(rays),
         "samples_per_s": round(W * H * SPP / dt, 1),
-        "roofline": trace_roofline(profiled_frame(ps, p, 0, 8), d),
+        "roofline": trace_roofline(profiled_frame(ps, p, 0, 8)),
     }
     if with_cpu:
         # the oracle on the same groom at 240x135 and 2 spp, scaled by
@@ -348,7 +347,7 @@ def textured(ctx, args, with_cpu):
         "ms_per_frame": round(dt * 1e3, 1),
         "mrays_per_s": round(rays / dt / 1e6, 1),
         "rays_per_frame": int(rays),
-        "roofline": trace_roofline(profiled_frame(ps, p, 0, 8), d),
+        "roofline": trace_roofline(profiled_frame(ps, p, 0, 8)),
     }
     ps.close()
     plain = scenes.pattern_zoo(W, H)
@@ -481,9 +480,9 @@ def time_to_relmse(ctx, args, with_cpu):
     ref.close()
     # rooflines from profiled (untimed) frames: plain frame 0; the cached
     # frame after 16 frames of training
-    plain["roofline"] = trace_roofline(profiled_frame(ps, params, 0, 4), d)
+    plain["roofline"] = trace_roofline(profiled_frame(ps, params, 0, 4))
     pn = profiled_frame(ps, params, 64, 4, nrc_config=rrhip.NrcConfig.make(), ctx=ctx)
-    nrc["roofline"] = trace_roofline(pn, d)
+    nrc["roofline"] = trace_roofline(pn)
     nrc["cache_kernels"] = cache_kernels(pn)
     out = {
         "workload": "instanced field 1920x1080 (10,000 x 20,480-triangle instances, 64 point + 1 rect light), "
@@ -579,7 +578,7 @@ def batched_jobs(ctx, args, with_cpu):
         "persistent": {"total_ms": round(pwall_ms, 2), "device_ms": round(ptotal_ms, 2),
                        "mrays_per_s": round(prays / (pwall_ms / 1e3) / 1e6, 1), "p50_ms": pct(pjob_ms, 50),
                        "p99_ms": pct(pjob_ms, 99), "launches": 1,
-                       "note": "one persistent launch: lanes pull (job, pixel) items shortest job first and "
+                       "note": "one persistent launch: waves pull chunks of pixels, shortest job first, and "
                                "regenerate paths in place; job completion from the device clock"},
         "rays": int(brays),
     }
