@@ -402,7 +402,10 @@ void tighten_bounds(const rrhip_scene_desc& d, const std::vector<BuiltBvh>& blas
   };
   const uint32_t nt = std::min({std::max(1u, std::thread::hardware_concurrency()), 16u, n / 256});
   std::vector<std::thread> th;
-  for (uint32_t k = 1; k < nt; k++) th.emplace_back(work);
+  try {
+    for (uint32_t k = 1; k < nt; k++) th.emplace_back(work);
+  } catch (const std::exception&) {  // no more threads to be had: those there are do the work
+  }
   work();
   for (std::thread& x : th) x.join();
 }
