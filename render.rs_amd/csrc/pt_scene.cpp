@@ -361,6 +361,32 @@ double camera_reach(const rrhip_camera_desc& c) {
   return r;
 }
 
+// Largest coordinate magnitude of the origin of a path's ray: on the camera,
+// on the geometry (`out`'s bounds, which do not count media), or where it
+// scattered in a medium. A density grid's box holds those points. Elsewhere
+// a run of up to 255 scatters can take the path away from everything, each
+// by as far as the transmittance is not zero in f32 (exp(-104)) and the
+// medium reaches, at most 1e8 (the segment of a ray that hits nothing).
+double origin_reach(const rrhip_scene_desc& d, const PtSceneHost& out) {
+  double reach = camera_reach(d.camera), step = 0.0;
+  for (int a = 0; a < 3; a++)
+    reach = std::max({reach, std::fabs((double)out.lo[a]), std::fabs((double)out.hi[a])});
+  for (uint32_t i = 0; i < d.num_media; i++) {
+    const rrhip_medium_desc& m = d.media[i];
+    if (m.nx > 0) {
+      for (int a = 0; a < 3; a++) reach = std::max({reach, std::fabs(m.grid_lo[a]), std::fabs(m.grid_hi[a])});
+      continue;
+    }
+    double thin = INFINITY;  // the smallest coefficient of a channel that scatters or absorbs
+    for (int c = 0; c < 3; c++)
+      if (m.sigma_a[c] + m.sigma_s[c] > 0.0) thin = std::min(thin, m.sigma_a[c] + m.sigma_s[c]);
+    double far = m.max_distance > 0.0 ? std::min(1e8, m.max_distance) : 1e8;
+    if (m.procedural == 0) far = std::min(far, 104.0 / thin);
+    step = std::max(step, far);
+  }
+  return reach + 255.0 * step;
+}
+
 // Calls work(i) for i in [0, n) from up to 16 threads, `chunk` at a time; the
 // calling thread does what no other can be started for.
 template <class F>
@@ -412,9 +438,12 @@ double map_support(const double* map, const double n[3]) {
 
 // Tight world bounds of the instances: the extent of the placed BLAS along
 // each world axis instead of its box's corners (a turned box is up to sqrt(3)
-// wider), padded by what the traversal's f32 mapping of a ray into object
-// space can move a hit (16 half-ulps of the largest ray coordinate taken
-// through the inverse and back), never wider than the corner box. With one
+// wider), padded by what f32 can move a ray that the placed BLAS's boxes
+// still accept, never wider than the corner box. In units of 2^-24 of the
+// largest coordinate of a ray's origin taken through the inverse and back:
+// 5 for mapping the origin (its matrix, products and sums), 4 of twice that
+// for mapping the direction, 3 of twice that for the slab test in either
+// space: 25, taken as 32. With one
 // instance per TLAS leaf, a closest-hit ray of the 10,000-instance field
 // (540p, depth 12) enters 1.9 instances instead of 10.6 and visits 55 nodes
 // instead of 66: frame 29.9 -> 22.1 ms. Six searches an instance cost 0.11 s
@@ -423,9 +452,7 @@ double map_support(const double* map, const double n[3]) {
 // instead (33 ms).
 void tighten_bounds(const rrhip_scene_desc& d, const std::vector<BuiltBvh>& blas, const std::vector<PtInstance>& raw,
                     const PtSceneHost& out, std::vector<float>& boxes) {
-  double reach = camera_reach(d.camera);
-  for (int a = 0; a < 3; a++)
-    reach = std::max({reach, std::fabs((double)out.lo[a]), std::fabs((double)out.hi[a])});
+  const double reach = origin_reach(d, out);
   // moving instances keep their corner boxes: the inverse varies over the shutter
   const auto placed = [&](uint32_t i) { return !blas[raw[i].mesh].nodes.empty() && !d.instances[i].moving; };
   std::vector<uint32_t> uses(blas.size(), 0), mapped;
@@ -458,7 +485,7 @@ void tighten_bounds(const rrhip_scene_desc& d, const std::vector<BuiltBvh>& blas
         const double o = std::fabs((double)v[0]) + std::fabs((double)v[1]) + std::fabs((double)v[2]);
         moved += std::fabs(M[k]) * (o * reach + std::fabs((double)v[3]));
       }
-      const double pad = moved * 9.5367431640625e-07;  // 2^-20
+      const double pad = moved * 1.9073486328125e-06;  // 2^-19
       float* b = &boxes[6 * (size_t)i];
       b[r] = std::max(b[r], std::nextafter((float)(lo - pad), -INFINITY));
       b[3 + r] = std::min(b[3 + r], std::nextafter((float)(hi + pad), INFINITY));

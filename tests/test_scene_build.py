@@ -114,25 +114,29 @@ def placed(count, kind, seed=3, moving=False, levels=2):
     return s, pos, idx
 
 
+def box_corners(tri):
+    """Corners of the boxes of triangles (n, 3, 3): (8, n, 3)."""
+    lo, hi = tri.min(1).astype(np.float64), tri.max(1).astype(np.float64)
+    return np.array([[(hi if k >> a & 1 else lo)[:, a] for a in range(3)] for k in range(8)]).transpose(0, 2, 1)
+
+
 # 168 uses search every bound, 170 go through the support map
 @pytest.mark.parametrize("count", [1, 168, 170, 400])
 @pytest.mark.parametrize("kind", ["turned", "axis", "sheared"])
 def test_instance_bounds_hold_and_are_tight(check, count, kind):
     s, pos, idx = placed(count, kind)
     boxes, fwd, _ = leaves(check, s.desc(max_leaf=1))
-    tri = pos[idx].astype(np.float64)
-    lo, hi = tri.min(1), tri.max(1)
-    corners = np.array([[(hi if k >> a & 1 else lo)[:, a] for a in range(3)] for k in range(8)]).transpose(0, 2, 1)
+    corners = box_corners(pos[idx])
     loose = []
     for b, f in zip(boxes, fwd.astype(np.float64)):
         p = pos @ f[:, :3].T + f[:, 3]
         rounded = (np.abs(f[:, :3]) @ np.abs(pos).max(0) + np.abs(f[:, 3])) * 2.0**-24  # f was read back as f32
         assert (b[0] <= p.min(0) + rounded).all() and (b[1] >= p.max(0) - rounded).all()
         # against the triangles' boxes: the pad (ray coordinates of at most
-        # 64, to object space and back, 2^-20 of them) and what the map adds
+        # 64, to object space and back, 2^-19 of them) and what the map adds
         inv = np.linalg.inv(f[:, :3])
         obj = np.abs(inv).sum(1) * 64 + np.abs(inv @ f[:, 3])
-        pad = (np.abs(f[:, 3]) + np.abs(f[:, :3]) @ obj) * 2.0**-20 + 1e-5
+        pad = (np.abs(f[:, 3]) + np.abs(f[:, :3]) @ obj) * 2.0**-19 + 1e-5
         q = corners @ f[:, :3].T + f[:, 3]
         radius = np.linalg.norm(f[:, :3], axis=1) * np.linalg.norm(pos, axis=1).max()
         loose.append((np.stack([q.min((0, 1)) - b[0], b[1] - q.max((0, 1))]) - pad) / radius)
@@ -140,6 +144,36 @@ def test_instance_bounds_hold_and_are_tight(check, count, kind):
     # cell's two edges of 1/6, so its chord is 1/12 above it at most
     assert np.max(loose) <= (2 / 12 if count > 169 else 0.0)
     assert np.mean(loose) <= 0.01
+
+
+MEDIA = {  # arguments of add_medium, and how far from everything a path scatters
+    "grid": (dict(sigma_a=(0.1,) * 3, sigma_s=(1, 1, 1), density=np.ones((2, 2, 2), np.float32),
+                  grid_lo=(-500, -2, -2), grid_hi=(2, 2, 2)), 500),
+    "near": (dict(sigma_a=(0, 0, 0), sigma_s=(0.01, 0, 0), max_distance=3.0), 60 + 255 * 3),
+    "dense": (dict(sigma_a=(1, 0, 1), sigma_s=(2, 0, 0.5)), 60 + 255 * 104 / 1.5),
+    "thin": (dict(sigma_a=(0, 0, 0), sigma_s=(1e-5,) * 3), 1e8),
+    "thin in one channel": (dict(sigma_a=(0, 0, 0), sigma_s=(1, 1, 1e-6)), 1e8),
+    "field": (dict(sigma_a=(0, 0, 0), sigma_s=(9, 9, 9), fbm={}), 1e8),
+}
+
+
+@pytest.mark.parametrize("kind", MEDIA)
+def test_instance_bounds_count_scatter_points(check, kind):
+    """Rays that start where a path scattered, far from all geometry, are
+    mapped into an instance with an error of 2^-19 of that distance; no box
+    may be padded by less, up to the corner box."""
+    s, pos, idx = placed(5, "turned")
+    medium, far = MEDIA[kind]
+    s.atmosphere = s.add_medium(**medium)
+    boxes, fwd, _ = leaves(check, s.desc(max_leaf=1))
+    corners, ends = box_corners(pos[idx]), box_corners(pos[None])[:, 0]
+    for b, f in zip(boxes, fwd.astype(np.float64)):
+        p, q = corners @ f[:, :3].T + f[:, 3], ends @ f[:, :3].T + f[:, 3]
+        pad = (np.abs(f[:, :3]) @ (np.abs(np.linalg.inv(f[:, :3])).sum(1) * far)) * 2.0**-19
+        assert (b[0] <= np.maximum(p.min((0, 1)) - pad, q.min(0)) + 1e-5).all()
+        assert (b[1] >= np.minimum(p.max((0, 1)) + pad, q.max(0)) - 1e-5).all()
+    if far < 1e3:  # and where no path gets far, the boxes stay tight
+        assert (boxes[:, 0] > (ends @ fwd[:, :, :3].transpose(0, 2, 1) + fwd[:, None, :, 3]).min(1) + 0.02).any()
 
 
 def test_bounds_cost_little():
