@@ -94,8 +94,9 @@ int check_build(const rrhip_scene_desc* d) {
 uint32_t check_stack_need() { return g_scene.stack_need; }
 
 // Per instance in leaf order: its leaf's box (lo, hi), its placement and
-// its geometry.
-void check_leaves(float* boxes, float* fwd, uint32_t* geometry) {
+// its geometry. Returns the most instances in a leaf.
+int check_leaves(float* boxes, float* fwd, uint32_t* geometry) {
+  uint32_t most = 0;
   std::vector<uint32_t> todo = {0};
   while (!todo.empty()) {
     const Node2 n = g_scene.nodes[todo.back()];
@@ -105,6 +106,7 @@ void check_leaves(float* boxes, float* fwd, uint32_t* geometry) {
     const uint32_t ref[2] = {n.ref0, n.ref1}, cnt[2] = {n.cnt0, n.cnt1};
     for (int k = 0; k < 2; k++) {
       if (cnt[k] == 0) todo.push_back(ref[k]);
+      most = std::max(most, cnt[k]);
       for (uint32_t i = ref[k]; i < ref[k] + cnt[k]; i++) std::memcpy(boxes + 6 * i, b[k], sizeof(b[k]));
     }
   }
@@ -112,6 +114,7 @@ void check_leaves(float* boxes, float* fwd, uint32_t* geometry) {
     std::memcpy(fwd + 12 * i, &g_scene.inst_fwd[12 * i], 12 * sizeof(float));
     geometry[i] = g_scene.insts[i].mesh;
   }
+  return (int)most;
 }
 
 // The most entries a lane's stack holds over `walks` traversals that hit

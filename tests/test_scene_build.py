@@ -71,13 +71,13 @@ def ptr(a, t=ctypes.c_float):
     return a.ctypes.data_as(ctypes.POINTER(t))
 
 
-def leaves(check, desc):
-    """(boxes, placements, geometries) of the built instances, leaf order."""
-    n = check.check_build(ctypes.byref(desc))
-    assert n >= 0
+def leaves(check, s, max_leaf):
+    """(boxes, placements, geometries) of the built instances of scene s in
+    leaf order, and the most in a leaf."""
+    n = check.check_build(ctypes.byref(s.desc(max_leaf=max_leaf)))
+    assert n == len(s.instances)
     boxes, fwd, geo = np.empty((n, 2, 3), np.float32), np.empty((n, 3, 4), np.float32), np.empty(n, np.uint32)
-    check.check_leaves(ptr(boxes), ptr(fwd), ptr(geo, ctypes.c_uint32))
-    return boxes, fwd, geo
+    return boxes, fwd, geo, check.check_leaves(ptr(boxes), ptr(fwd), ptr(geo, ctypes.c_uint32))
 
 
 @pytest.mark.parametrize("bins,max_leaf", [(2, 1), (32, 1), (32, 4), (7, 2), (32, 8)])
@@ -125,7 +125,7 @@ def box_corners(tri):
 @pytest.mark.parametrize("kind", ["turned", "axis", "sheared"])
 def test_instance_bounds_hold_and_are_tight(check, count, kind):
     s, pos, idx = placed(count, kind)
-    boxes, fwd, _ = leaves(check, s.desc(max_leaf=1))
+    boxes, fwd, _, _ = leaves(check, s, 1)
     corners = box_corners(pos[idx])
     loose = []
     for b, f in zip(boxes, fwd.astype(np.float64)):
@@ -165,7 +165,7 @@ def test_instance_bounds_count_scatter_points(check, kind):
     s, pos, idx = placed(5, "turned")
     medium, far = MEDIA[kind]
     s.atmosphere = s.add_medium(**medium)
-    boxes, fwd, _ = leaves(check, s.desc(max_leaf=1))
+    boxes, fwd, _, _ = leaves(check, s, 1)
     corners, ends = box_corners(pos[idx]), box_corners(pos[None])[:, 0]
     for b, f in zip(boxes, fwd.astype(np.float64)):
         p, q = corners @ f[:, :3].T + f[:, 3], ends @ f[:, :3].T + f[:, 3]
@@ -191,3 +191,56 @@ def test_bounds_cost_little():
             best = min(best, time.process_time() - t)
         return best
     assert cpu(False) < 2.0 * cpu(True)
+
+
+def chain(count, ratio, links):
+    """`count` instances, each `ratio` of the one before it in size and in
+    distance from the origin, of a mesh of `links` triangles in a row of the
+    same kind: binned splits peel such rows from one end, so the trees are
+    deep."""
+    s = scenes.Scene(8, 8, 45.0, eye=(0, 0, -9), look_at=(0, 0, 0))
+    m = s.add_material(scenes.matte((0.5, 0.5, 0.5)))
+    tri = np.array([[0, 0, 0], [0.3, 0, 0], [0, 0.3, 0.1]])
+    pos = np.concatenate([(tri + (2, 0, 0)) * x for x in 0.7**np.arange(links)]).astype(np.float32)
+    mesh = s.add_mesh(pos, np.arange(3 * links, dtype=np.uint32).reshape(-1, 3))
+    for x in ratio ** np.arange(count, dtype=np.float64):
+        s.add_instance(mesh, m, np.hstack([np.diag([0.1 * x] * 3), [[3 * x], [0], [0]]]))
+    return s
+
+
+# (instances, ratio, links, max_leaf): stacks well below, at and above the 32
+# and 48 entries of the kernels' columns; then hierarchies whose tree of
+# single instances outgrows the stack, so that the shallower tree over
+# corner boxes and leaves of up to 8 is taken; then one too deep either way
+DEEP = [(1, 0.5, 1, 1), (1, 0.5, 40, 1), (5, 0.5, 8, 4), (30, 0.5, 8, 1), (43, 0.4, 20, 1), (46, 0.4, 20, 1), (60, 0.4, 40, 1),
+        (60, 0.4, 40, 8), (90, 0.4, 1, 4), (90, 0.4, 8, 8), (90, 0.4, 40, 8), (86, 0.35, 8, 8), (88, 0.35, 20, 8),
+        (110, 0.4, 40, 4)]
+
+
+@pytest.mark.parametrize("count,ratio,links,max_leaf", DEEP)
+def test_stack_need_covers_every_traversal(check, count, ratio, links, max_leaf):
+    most = leaves(check, chain(count, ratio, links), max_leaf)[3]
+    need = check.check_stack_need()
+    use = max(check.check_stack_use(100, miss, count) for miss in (0.0, 0.1, 0.3, 0.6))
+    assert use <= need
+    if count in (86, 88):
+        assert most > 1 and need <= 48
+    elif need <= 48:
+        assert most == 1  # an exact need, which a traversal reaches unless the deepest parts exclude each other
+        assert use >= need - 9
+
+
+def test_deep_cases_reach_the_column_sizes(check):
+    need = []
+    for count, ratio, links, max_leaf in DEEP:
+        leaves(check, chain(count, ratio, links), max_leaf)
+        need.append(check.check_stack_need())
+    assert min(need) == 2 and 32 in need and 33 in need and 48 in need and max(need) > 48, need
+
+
+@pytest.mark.parametrize("max_leaf", [1, 4, 8])
+def test_stack_need_of_scattered_instances(check, max_leaf):
+    for count in (2, 3, 9, 500):
+        leaves(check, placed(count, "sheared", seed=count)[0], max_leaf)
+        use = max(check.check_stack_use(100, miss, count) for miss in (0.0, 0.1, 0.3))
+        assert check.check_stack_need() - 2 <= use <= check.check_stack_need()
