@@ -46,8 +46,9 @@ hipError_t pt_launch_bounce(const PtSceneView& S, PathBuffers P, const PtParams&
 hipError_t pt_launch_last_shadows(const PtSceneView& S, const PathBuffers& P, uint32_t capacity, hipStream_t st);
 // The trace kernels, with gt blocks: closest hits of the live queue `q` of
 // P.round (kTraceExtend), visibility of the shadow records that the round
-// before wrote (kTraceShadow), or both in one launch (kTraceRound: opaque
-// scenes, not while profiling).
+// before wrote (kTraceShadow; q is not used), or both in one launch
+// (kTraceRound: opaque scenes, not while profiling; others are refused with
+// hipErrorInvalidValue, as is a missing queue).
 enum TraceWork { kTraceExtend, kTraceShadow, kTraceRound };
 hipError_t pt_launch_trace(const PtSceneView& S, const PathBuffers& P, const uint32_t* q, uint32_t gt, TraceWork work,
                            hipStream_t st);

@@ -424,7 +424,7 @@ hipError_t pt_launch_bounce(const PtSceneView& S, PathBuffers P, const PtParams&
 
 hipError_t pt_launch_last_shadows(const PtSceneView& S, const PathBuffers& P, uint32_t capacity, hipStream_t st) {
   if (P.prof || S.transparent) return hipSuccess;
-  return pt_launch_trace(S, P, nullptr, trace_grid(capacity), kTraceRound, st);
+  return pt_launch_trace(S, P, nullptr, trace_grid(capacity), kTraceShadow, st);
 }
 
 hipError_t pt_launch_batch_pass(const PtJob* jobs, uint32_t nj, PathBuffers P, uint32_t total,
