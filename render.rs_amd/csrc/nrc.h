@@ -88,11 +88,14 @@ hipError_t nrc_launch_update(const NrcGridView& G, const float* part, NrcControl
 hipError_t nrc_launch_reduce_mlp(const float* part, NrcControl* ctl, uint32_t capacity, float* w, float* m,
                                  float* v, float* grad_out, NrcHyper hp, bool apply, hipStream_t st);
 // Adam on the grid with the moving average ema = alpha ema + (1 - alpha)
-// table and its debiased value (step ctl->t) into `inf`; without `apply`
-// the grid gradient as f32 into grad_out. Clears the gradients.
-hipError_t nrc_launch_adam_grid(float* table, float* m, float* v, unsigned long long* grid_grad, uint8_t* touched,
-                                uint64_t n, const NrcControl* ctl, float* grad_out, NrcHyper hp, bool apply,
-                                hipStream_t st, float* ema = nullptr, float* inf = nullptr, float alpha = 0.f);
+// table and its debiased value (step ctl->t) into `inf`; clears the
+// gradients.
+hipError_t nrc_launch_adam_grid_ema(float* table, float* m, float* v, unsigned long long* grid_grad, uint8_t* touched,
+                                    uint64_t n, const NrcControl* ctl, NrcHyper hp, float* ema, float* inf, float alpha,
+                                    hipStream_t st);
+// The grid gradient as f32 into grad_out; clears the gradients.
+hipError_t nrc_launch_grid_gradient(unsigned long long* grid_grad, uint8_t* touched, uint64_t n, const NrcControl* ctl,
+                                    float* grad_out, hipStream_t st);
 // The same moving average over the MLP master weights (when ctl->n > 0).
 hipError_t nrc_launch_ema_mlp(const float* w, float* ema, float* inf, const NrcControl* ctl, float alpha,
                               hipStream_t st);

@@ -659,29 +659,39 @@ __device__ __forceinline__ float ema_debias(const NrcControl* ctl, float a) {
   return (float)(1.0 / (1.0 - pow((double)a, (double)ctl->t)));
 }
 
-// The grid's update with a moving average for inference (apply), or its
-// gradient alone; clears the gradients.
-__global__ __launch_bounds__(256) void nrc_adam_grid_kernel(float* __restrict__ table, float* __restrict__ m,
-                                                           float* __restrict__ v, unsigned long long* __restrict__ gg,
-                                                           uint8_t* __restrict__ touched, uint64_t n,
-                                                           const NrcControl* __restrict__ ctl,
-                                                           float* __restrict__ grad_out, NrcHyper hp, int apply,
-                                                           float* __restrict__ ema, float* __restrict__ inf,
-                                                           float alpha) {
+// The waiting gradient of grid parameter i as f32; clears it and its mark.
+__device__ __forceinline__ float take_grad(unsigned long long* __restrict__ gg, uint8_t* __restrict__ touched, uint64_t i) {
+  const long long fx = (long long)gg[i];
+  if (fx != 0) gg[i] = 0ull;
+  if ((i & 3u) == 0) touched[i >> 2] = 0;
+  return (float)fx * (1.f / 68719476736.f);
+}
+
+__global__ __launch_bounds__(256) void nrc_grid_gradient_kernel(unsigned long long* __restrict__ gg,
+                                                               uint8_t* __restrict__ touched, uint64_t n,
+                                                               const NrcControl* __restrict__ ctl,
+                                                               float* __restrict__ grad_out) {
   if (ctl->n == 0) return;
-  float c1 = 1.f, c2 = 1.f;
-  if (apply) bias_corrections(ctl, hp, c1, c2);
-  const float corr = ema ? ema_debias(ctl, alpha) : 1.f;
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+    grad_out[i] = take_grad(gg, touched, i);
+}
+
+// The grid's update with a moving average for inference.
+__global__ __launch_bounds__(256) void nrc_adam_grid_ema_kernel(float* __restrict__ table, float* __restrict__ m,
+                                                               float* __restrict__ v,
+                                                               unsigned long long* __restrict__ gg,
+                                                               uint8_t* __restrict__ touched, uint64_t n,
+                                                               const NrcControl* __restrict__ ctl, NrcHyper hp,
+                                                               float* __restrict__ ema, float* __restrict__ inf,
+                                                               float alpha) {
+  if (ctl->n == 0) return;
+  float c1, c2;
+  bias_corrections(ctl, hp, c1, c2);
+  const float corr = ema_debias(ctl, alpha);
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const long long fx = (long long)gg[i];
-    if (fx != 0) gg[i] = 0ull;
-    if ((i & 3u) == 0) touched[i >> 2] = 0;
-    const float g = (float)fx * (1.f / 68719476736.f);
-    if (!apply) {
-      grad_out[i] = g;
-      continue;
-    }
+    const float g = take_grad(gg, touched, i);
     float p = table[i], mm = m[i], vv = v[i];
     adam_update(p, g, mm, vv, hp, c1, c2);
     table[i] = p;
@@ -801,13 +811,23 @@ hipError_t nrc_launch_update(const NrcGridView& G, const float* part, NrcControl
   return hipGetLastError();
 }
 
-hipError_t nrc_launch_adam_grid(float* table, float* m, float* v, unsigned long long* grid_grad, uint8_t* touched,
-                                uint64_t n, const NrcControl* ctl, float* grad_out, NrcHyper hp, bool apply,
-                                hipStream_t st, float* ema, float* inf, float alpha) {
+static uint32_t grid_blocks(uint64_t n) {
   const uint64_t b = (n + 255) / 256;
-  const uint32_t blocks = (uint32_t)(b > 8192 ? 8192 : (b < 1 ? 1 : b));
-  hipLaunchKernelGGL(nrc_adam_grid_kernel, dim3(blocks), dim3(256), 0, st, table, m, v, grid_grad, touched, n, ctl,
-                     grad_out, hp, apply ? 1 : 0, ema, inf, alpha);
+  return (uint32_t)(b > 8192 ? 8192 : (b < 1 ? 1 : b));
+}
+
+hipError_t nrc_launch_grid_gradient(unsigned long long* grid_grad, uint8_t* touched, uint64_t n, const NrcControl* ctl,
+                                    float* grad_out, hipStream_t st) {
+  hipLaunchKernelGGL(nrc_grid_gradient_kernel, dim3(grid_blocks(n)), dim3(256), 0, st, grid_grad, touched, n, ctl,
+                     grad_out);
+  return hipGetLastError();
+}
+
+hipError_t nrc_launch_adam_grid_ema(float* table, float* m, float* v, unsigned long long* grid_grad, uint8_t* touched,
+                                    uint64_t n, const NrcControl* ctl, NrcHyper hp, float* ema, float* inf, float alpha,
+                                    hipStream_t st) {
+  hipLaunchKernelGGL(nrc_adam_grid_ema_kernel, dim3(grid_blocks(n)), dim3(256), 0, st, table, m, v, grid_grad, touched,
+                     n, ctl, hp, ema, inf, alpha);
   return hipGetLastError();
 }
 

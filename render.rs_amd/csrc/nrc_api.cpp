@@ -147,8 +147,8 @@ hipError_t nrc_step_device(rrhip_nrc* c, const NrcQuery* q, const float* targets
   if (e == hipSuccess)
     e = nrc_launch_reduce_mlp(c->d_part, c->d_ctl, capacity, c->d_w, c->d_wm, c->d_wv, nullptr, c->hp, true, st);
   if (e == hipSuccess)
-    e = nrc_launch_adam_grid(c->d_table, c->d_tm, c->d_tv, c->d_tg, c->d_touched, c->grid_n, c->d_ctl, nullptr, c->hp,
-                             true, st, c->d_ema_table, c->d_inf_table, c->cfg.ema);
+    e = nrc_launch_adam_grid_ema(c->d_table, c->d_tm, c->d_tv, c->d_tg, c->d_touched, c->grid_n, c->d_ctl, c->hp,
+                                 c->d_ema_table, c->d_inf_table, c->cfg.ema, st);
   if (e == hipSuccess) e = nrc_launch_ema_mlp(c->d_w, c->d_ema_w, c->d_inf_w, c->d_ctl, c->cfg.ema, st);
   if (e == hipSuccess) e = nrc_launch_pack(c->d_inf_w, c->d_inf_wf, nullptr, c->d_ctl, false, st);
   if (e == hipSuccess) e = nrc_launch_pack(c->d_w, c->d_wf, c->d_wb, c->d_ctl, true, st);
@@ -376,8 +376,7 @@ int rrhip_nrc_gradients(rrhip_nrc* c, const rrhip_nrc_query* queries, const floa
                                  c->d_touched, st));
   RRHIP_HIP_TRY(nrc_launch_reduce_mlp(c->d_part, c->d_ctl, (uint32_t)n, c->d_w, c->d_wm, c->d_wv, c->d_wgrad, c->hp,
                                       false, st));
-  RRHIP_HIP_TRY(nrc_launch_adam_grid(c->d_table, c->d_tm, c->d_tv, c->d_tg, c->d_touched, c->grid_n, c->d_ctl,
-                                     c->d_gout, c->hp, false, st));
+  RRHIP_HIP_TRY(nrc_launch_grid_gradient(c->d_tg, c->d_touched, c->grid_n, c->d_ctl, c->d_gout, st));
   if (mlp_grad)
     RRHIP_HIP_TRY(hipMemcpyAsync(mlp_grad, c->d_wgrad, kNrcMlpParams * sizeof(float), hipMemcpyDeviceToHost, st));
   if (grid_grad)
