@@ -53,6 +53,45 @@ def test_cloud_tail_equals_rounds(width, height, spp, depth, film):
         ps.close()
 
 
+def entering(ps, p, depth, cache=None):
+    """Paths that enter bounce round `depth` of a pass, as the rounds count them."""
+    n = []
+    for d in (depth, depth + 1):
+        q = rrhip.RenderParams.make(max_depth=d, rr_start=p.rr_start, samples_per_pass=p.samples_per_pass)
+        n.append(render(ps, q, False, True, cache=cache)[2])
+    return n[1] - n[0]
+
+
+# more paths than the tails of rounds 4, 8 and 12 take (roulette starts
+# late): the tail of round 16 takes them all, about 30 to 100 a wave
+@pytest.mark.parametrize("width,height,spp,depth,rr_start", [(257, 256, 1, 17, 64), (400, 300, 1, 24, 64),
+                                                             (300, 230, 3, 64, 18)])
+@pytest.mark.parametrize("film", [False, True])
+def test_cloud_tail_takes_any_number_of_paths(width, height, spp, depth, rr_start, film):
+    s = scenes.cloud_room(width, height, n=16, sigma_s=(20.0,) * 3, sigma_a=(0.0,) * 3)
+    p = rrhip.RenderParams.make(max_depth=depth, rr_start=rr_start, samples_per_pass=spp)
+    with rrhip.Context(0) as ctx:
+        ps = rrhip.PtScene(ctx, s.desc())
+        assert entering(ps, p, 16) > 65536
+        ref = render(ps, p, film, True, passes=3)
+        for mode in (0, 1, 2):
+            same(render(ps, p, film, False, mode, passes=3), ref)
+        ps.close()
+
+
+@pytest.mark.parametrize("width,height,depth", [(300, 230, 17), (320, 240, 40)])
+def test_cache_tail_takes_any_number_of_paths(width, height, depth):
+    s = scenes.box_room(width, height)
+    p = rrhip.RenderParams.make(max_depth=depth, rr_start=64, samples_per_pass=2)
+    cfg = rrhip.NrcConfig.make(log2_table=14, train_paths=2048, batch=1024, spread=1e4)
+    with rrhip.Context(0) as ctx:
+        ps = rrhip.PtScene(ctx, s.desc())
+        # some paths have ended in a cache query by then, others do so in the tail
+        assert 65536 < entering(ps, p, 16, cfg) < 0.9 * (2 * width * height + 2048)
+        same(render(ps, p, False, False, passes=3, cache=cfg), render(ps, p, False, True, passes=3, cache=cfg))
+        ps.close()
+
+
 @pytest.mark.parametrize("width,height,depth", [(9, 7, 20), (320, 210, 12)])
 def test_cache_tail_equals_rounds(width, height, depth):
     s = scenes.box_room(width, height)
