@@ -65,7 +65,7 @@ struct rrhip_session {
   // accumulator (kFilmStride doubles per pixel) here.
   bool film = false;
   double* d_film = nullptr;
-  double* d_film_image = nullptr;  // channels of kFilmImageRows pixels, allocated by the first read
+  double* d_film_image = nullptr;  // channels of up to kFilmImageRows pixels, for rrhip_read_film
   // Profiling (rrhip_session_set_profiling): counting trace kernels whose
   // fetch totals land in prof_counts, events around each bounce's kernels
   // and the cache's inference and optimiser steps, device times summed per
@@ -550,14 +550,19 @@ int rrhip_session_set_film(rrhip_session* s, int enable) {
   hipError_t e = alloc_paths(s, s->path_cap);
   const uint64_t fbytes = (uint64_t)s->prm.npix * kFilmStride * sizeof(double);
   if (e == hipSuccess && s->film) e = hipMalloc((void**)&s->d_film, fbytes);
+  // here and not by the first read, which must not fail after a long render
+  const uint64_t ibytes = (uint64_t)std::min(s->prm.npix, kFilmImageRows) * kFilmChannels * sizeof(double);
+  if (e == hipSuccess && s->film) e = hipMalloc((void**)&s->d_film_image, ibytes);
   if (e == hipSuccess && s->film) e = hipMemsetAsync(s->d_film, 0, fbytes, s->scene->ctx->stream);
   if (e == hipSuccess && s->film) e = hipStreamSynchronize(s->scene->ctx->stream);
   if (e != hipSuccess) {
     // leave a usable plain session behind
     (void)hipGetLastError();
     s->film = false;
-    if (s->d_film) (void)hipFree(s->d_film);
-    s->d_film = nullptr;
+    for (double** p : {&s->d_film, &s->d_film_image}) {
+      if (*p) (void)hipFree(*p);
+      *p = nullptr;
+    }
     if (alloc_paths(s, s->path_cap) != hipSuccess) return fail_hip(e, "rrhip_session_set_film (session unusable)");
     return fail_hip(e, "rrhip_session_set_film");
   }
@@ -572,7 +577,6 @@ int rrhip_read_film(rrhip_session* s, double* out) {
   static_assert(kFilmChannels == RRHIP_FILM_CHANNELS, "film channels");
   const uint32_t npix = s->prm.npix, rows = std::min(npix, kFilmImageRows);
   hipStream_t st = s->scene->ctx->stream;
-  if (!s->d_film_image) RRHIP_HIP_TRY(hipMalloc((void**)&s->d_film_image, (uint64_t)rows * kFilmChannels * sizeof(double)));
   for (uint32_t p = 0; p < npix; p += rows) {
     const uint32_t n = std::min(rows, npix - p);
     RRHIP_HIP_TRY(pt_launch_film_image(s->d_accum + (uint64_t)p * RRHIP_ACCUM_STRIDE, s->d_film + (uint64_t)p * kFilmStride,

@@ -2,6 +2,7 @@
 pixel counts around the block size and past one launch's pixels."""
 import numpy as np
 import pytest
+import torch
 
 import rrhip
 import scenes
@@ -29,4 +30,23 @@ def test_film_channels_follow_the_accumulator(width, height):
             assert np.isin(f[:, 17], [0.0, 0.5, 1.0]).all()
             assert (f[:, 15] > 0).any()
         se.close()
+        ps.close()
+
+
+def test_reading_the_film_takes_no_device_memory():
+    """Film mode's buffers are there when it is switched on: a read after a
+    long render must not fail for want of memory (38 MB at this size)."""
+    s = scenes.box_room(513, 512)
+    p = rrhip.RenderParams.make(max_depth=1, samples_per_pass=1)
+    with rrhip.Context(0) as ctx:
+        ps = rrhip.PtScene(ctx, s.desc())
+        for first in (True, False):  # the first session's read loads the kernel's code
+            se = ps.session(p)
+            se.set_film(True)
+            se.render(0, 1)
+            free = torch.cuda.mem_get_info(0)[0]
+            se.film()
+            if not first:
+                assert torch.cuda.mem_get_info(0)[0] == free
+            se.close()
         ps.close()
