@@ -297,8 +297,9 @@ namespace {
 hipError_t persistent_setup(rrhip_batch* b) {
   if (b->d_pjobs) return hipSuccess;
   const uint32_t nj = (uint32_t)b->jobs.size();
-  bool eq = false;
+  bool eq = false, chunks = false;  // chunks: some job's samples wait for their chunk's end
   for (const rrhip_batch_job& J : b->jobs) {
+    chunks |= J.spp <= kPtChunkSamples;
     b->p_flags |= (J.scene->pt.transparent ? 1u : 0u) | (J.scene->pt.motion ? 2u : 0u) |
                   (J.scene->pt.num_quadrics || J.scene->pt.curves ? 4u : 0u);
     eq |= J.scene->pt_eq;
@@ -337,7 +338,7 @@ hipError_t persistent_setup(rrhip_batch* b) {
   if (e == hipSuccess) e = alloc_n(b, &b->d_next, 1);
   if (e == hipSuccess) e = alloc_n(b, &b->d_left, nj);
   if (e == hipSuccess) e = alloc_n(b, &b->d_clock, (uint64_t)nj + 1);
-  if (e == hipSuccess) e = alloc_n(b, &b->d_samples, n * kPtChunkSamples);
+  if (e == hipSuccess && chunks) e = alloc_n(b, &b->d_samples, n * kPtChunkSamples);
   if (e == hipSuccess) e = alloc_n(b, &b->d_pjobs, nj);
   return e;
 }

@@ -3,6 +3,7 @@ its waves' lanes: at samples per pixel around a chunk's 64 and pixel counts
 that leave a remainder, every job equals its own session bit for bit."""
 import numpy as np
 import pytest
+import torch
 
 import rrhip
 import scenes
@@ -35,3 +36,22 @@ def test_every_job_equals_its_session(jobs):
         b.close()
         for ps, _, _ in work:
             ps.close()
+
+
+@pytest.mark.parametrize("spp,least,most", [(64, 100, 400), (65, 0, 100)])
+def test_sample_scratch_only_where_samples_wait(spp, least, most):
+    """Jobs of more than 64 samples a pixel add them one by one: the first
+    persistent launch of such a batch takes none of the 134 MB in which the
+    others' samples wait."""
+    s = scenes.box_room(8, 8)
+    p = rrhip.RenderParams.make(max_depth=2)
+    with rrhip.Context(0) as ctx:
+        ps = rrhip.PtScene(ctx, s.desc())
+        for first in (True, False):  # the first batch loads the kernel's code
+            b = rrhip.Batch(ctx, [(ps, spp, p)])
+            free = torch.cuda.mem_get_info(0)[0]
+            b.render_persistent()
+            taken = (free - torch.cuda.mem_get_info(0)[0]) >> 20
+            b.close()
+        assert least <= taken <= most, taken
+        ps.close()
