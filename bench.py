@@ -91,7 +91,9 @@ def cpu_baseline(pos, idx, rays):
 # 48-byte triangle records, 80 bytes per instance entered (instance and
 # mesh records). The loose objects, which every ray tests, are a few KB that
 # the nearest caches hold and count nothing: with them a box room's 22
-# would move 18.8 TB/s.
+# would move 18.8 TB/s. Most of the other fetches are served by L2 and the
+# Infinity Cache as well (0.96 of the instanced field's), so the model's rate
+# over the HBM peak says how much the kernels ask for, not what memory moves.
 EXTEND_STATE_BYTES = 4 + 32 + 52   # queue entry; origin, direction; hit normal/t, material, two origins
 SHADOW_STATE_BYTES = 4 + 48 + 32   # queue entry; origin, direction, contribution; radiance read + write
 HBM_PEAK = 8000.0  # GB/s
@@ -122,8 +124,10 @@ def trace_roofline(prof):
             "frac": round(achieved / HBM_PEAK, 4), "traffic": None,
             "kernels": {"extend": ext, "shadow": sh, "shade_ms": round(prof["shade_ms"], 3)},
             "note": "extend + shadow kernels over one profiled frame: B-model bytes (path state, node / "
-                    "triangle / instance fetches counted by the profiling kernels) over their event-timed "
-                    "device time"}
+                    "triangle / instance fetches counted by the profiling kernels, most of them served by "
+                    "caches) over their event-timed device time; a profiled frame traces closest hits and "
+                    "shadow rays in launches of their own and runs every round, an unprofiled one merges "
+                    "the two in opaque scenes and ends clouds and cache passes in a tail launch"}
 
 
 def profiled_frame(ps, params, start, count, nrc_config=None, ctx=None):

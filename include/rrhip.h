@@ -654,7 +654,12 @@ int rrhip_read_film(rrhip_session* session, double* out);
  * of the trace kernels (same results) and times each bounce's kernels and
  * the radiance cache's work with device events, waiting for each pass
  * (graph replay is off meanwhile); the profile starts empty now. 0 turns
- * it off. No counterpart in render.rs; it feeds the traversal bytes model
+ * it off. A profiled pass is a wavefront with a launch per kind of work: it
+ * traces closest hits and shadow rays apart, where an opaque scene's pass
+ * otherwise traces a round's shadow rays with the next round's closest hits,
+ * and runs every round, where a cloud's or a cache's pass otherwise ends in
+ * a launch that finishes the last paths. Fetch and ray counts are those of
+ * any pass; times are this one's. No counterpart in render.rs; it feeds the traversal bytes model
  * of the path-tracing benchmarks. */
 typedef struct rrhip_pt_profile {
   uint64_t extend_rays, extend_nodes, extend_triangles, extend_instances;

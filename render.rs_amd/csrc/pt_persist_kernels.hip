@@ -26,7 +26,7 @@ constexpr uint32_t kOpenChunks = 64;  // chunks a wave can have open at once
 // the last chunk and its paths are done.
 //
 // Bound by latency at two waves per SIMD (the registers of media shading)
-// and 20 lanes per vector instruction. With a pixel and all its samples per
+// and 25 lanes per vector instruction. With a pixel and all its samples per
 // lane, the lanes that drew the last pixels of the longest job ran up to 16
 // paths one after another while the others had ended, and the lanes of a
 // wave drifted apart into different jobs: 16 rooms of up to 256 x 256

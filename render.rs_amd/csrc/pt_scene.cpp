@@ -443,13 +443,14 @@ double map_support(const double* map, const double n[3]) {
 // largest coordinate of a ray's origin taken through the inverse and back:
 // 5 for mapping the origin (its matrix, products and sums), 4 of twice that
 // for mapping the direction, 3 of twice that for the slab test in either
-// space: 25, taken as 32. With one
-// instance per TLAS leaf, a closest-hit ray of the 10,000-instance field
-// (540p, depth 12) enters 1.9 instances instead of 10.6 and visits 55 nodes
-// instead of 66: frame 29.9 -> 22.1 ms. Six searches an instance cost 0.11 s
-// of processor time there (build 30 -> 51 ms with 8 threads); a geometry
-// placed more often than its support map takes searches goes through the map
-// instead (33 ms).
+// space: 25, taken as 32.
+//
+// With one instance per TLAS leaf, a closest-hit ray of the 10,000-instance
+// field (540p, depth 12) enters 1.9 instances instead of 10.6 and visits 55
+// nodes instead of 66: 29.9 -> 22.1 ms of device time a frame. Six searches an
+// instance cost 0.11 s of processor time there (build 30 -> 51 ms with 8
+// threads); a geometry placed more often than its support map takes searches
+// goes through the map instead (33 ms).
 void tighten_bounds(const rrhip_scene_desc& d, const std::vector<BuiltBvh>& blas, const std::vector<PtInstance>& raw,
                     const PtSceneHost& out, std::vector<float>& boxes) {
   const double reach = origin_reach(d, out);

@@ -16,8 +16,8 @@ using namespace pt;
 // the surface lobes to 218-228 registers, and under a three-wave cap it
 // spilled 96 to 168 B per lane to scratch in every scene; scenes without
 // media therefore have kernels of their own, the others run two waves
-// without spills (200 x 200 cloud room, 16 samples: frame 4.98 -> 4.48 ms;
-// 256 x 256 box room: 1.19 -> 1.08 ms).
+// without spills (200 x 200 cloud room, 16 samples: 4.98 -> 4.48 ms of
+// device time a frame; 256 x 256 box room: 1.19 -> 1.08).
 template <bool NRC, bool TR, bool MEDIA, bool FILM = false, bool FIXED = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(MEDIA ? 2 : 3))) void shade_kernel(
     PtSceneView S, PathBuffers P, PtParams prm, const uint32_t* __restrict__ q, uint32_t* __restrict__ qnext,

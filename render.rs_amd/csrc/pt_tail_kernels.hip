@@ -20,9 +20,9 @@ using namespace pt;
 // tenth of the paths. Here a pass waits once for its longest path instead of
 // once a round. Two waves per SIMD, so that shading does not spill; a wave
 // refills its idle lanes from its run of the queue. 200 x 200 cloud room, 16
-// samples, 64 bounces: 3.90 -> 3.10 ms a frame (300 x 290: 5.87 -> 4.97,
-// 150 x 140 with 3 samples: 1.98 -> 1.39); 960 x 540 instanced field through
-// the radiance cache, 4 samples, 12 bounces: 8.45 -> 7.91 ms.
+// samples, 64 bounces: 3.90 -> 3.10 ms of device time a frame (300 x 290:
+// 5.87 -> 4.97, 150 x 140 with 3 samples: 1.98 -> 1.39); 960 x 540 instanced
+// field through the radiance cache, 4 samples, 12 bounces: 8.45 -> 7.91.
 template <bool NRC, bool MEDIA, bool FILM>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(2))) void tail_kernel(
     PtSceneView S, PathBuffers P, PtParams prm, const uint32_t* __restrict__ q, NrcPathBuffers N, uint32_t limit) {

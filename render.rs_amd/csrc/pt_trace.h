@@ -21,7 +21,8 @@ namespace pt {
 // Stack entry of a TLAS leaf still to enter: flag, count - 1 (bits 28-30),
 // first instance (bits 0-27). One entry per leaf keeps the TLAS phase at
 // one entry per level (two at the last), so a lane needs at most
-// tlas_levels + blas_levels + 2 entries.
+// tlas_levels + blas_levels + 2 entries; the host build counts what the two
+// trees really need (tlas_stack, blas_stack).
 constexpr uint32_t kInstEntry = 0x80000000u;
 constexpr uint32_t kInstFirst = 0x0FFFFFFFu;
 
@@ -164,13 +165,14 @@ __device__ __forceinline__ void instance_inverse(const PtSceneView& S, const PtI
 // instruction on the 10,000-instance field (540p, 8 samples) and 6 on the
 // 300,000-segment fur ball (360p, 8 samples), at 0.7 and 0.5 of the issue
 // slots. Voted steps run 23 and 16 lanes: 32 and 40 % fewer vector
-// instructions, fur ball frame 31.3 -> 21.4 ms, field 30.7 -> 29.9 ms (and
-// 22.1 ms with the tight instance bounds that cut its instance entries).
+// instructions, fur ball 31.3 -> 21.4 ms of device time a frame, field 30.7
+// -> 29.9 (and 22.1 with the tight instance bounds that cut its instance
+// entries).
 // Counting the votes as two 32-bit halves, in scalar registers, and keeping
 // the hit's distance and flag only in tmax and hit.inst, took the field's
 // trace and shade launches from 16.1 to 15.2 ms and the ball's from 13.2 to
-// 12.9. Each lane's own order of visits and tests is unchanged, and so are
-// the hits. Slower: waiting for 20 lanes before a leaf or instance step instead
+// 12.9. The vote changes no lane's own order of visits and tests, and so no
+// hit. Slower: waiting for 20 lanes before a leaf or instance step instead
 // of the vote (field 33.7 ms); a step of its own for the segments' f64 test
 // (fur ball +15 %); refilling done lanes from the queue (field +13 %).
 template <int STRIDE, bool ANY, bool MOTION, bool COUNT, bool CURVES>

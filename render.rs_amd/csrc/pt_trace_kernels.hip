@@ -58,9 +58,9 @@ __global__ __launch_bounds__(kTraceBlock) void shadow_kernel(PtSceneView S, Path
 // under the closest hits' end instead of after it. Extension rays, the
 // longer ones, come first. A wave's lanes all hold the same kind of ray.
 // Without a queue (q null) only the shadow records are traced.
-// With the counter rotation's launch gone as well: 540p instanced field 18.6
-// -> 16.1 ms a frame, 200 x 200 cloud room 4.46 -> 3.88 ms, 256 x 256 box
-// room 1.08 -> 1.02 ms.
+// With the counter rotation's launch gone as well, device time a frame: 540p
+// instanced field 18.6 -> 16.1 ms, 200 x 200 cloud room 4.46 -> 3.88, 256 x
+// 256 box room 1.08 -> 1.02.
 template <int STACK, bool MOTION, int GEO>
 __global__ __launch_bounds__(kTraceBlock) void trace_kernel(PtSceneView S, PathBuffers P, const uint32_t* __restrict__ q) {
   constexpr int SG = GEO & ~kGeoSt;  // shadow rays need no texture coordinates

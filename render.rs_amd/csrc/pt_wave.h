@@ -63,7 +63,8 @@ __device__ __forceinline__ void stack_pop(uint32_t& depth) {
 // appends at the same addresses, where an update takes about 10 ns, so one
 // atomic per wave and queue bounded the shade pass: a 256 x 256 room at 16
 // samples (up to 16,384 waves a pass, 7 % of the vector issue slots used)
-// took 211 us a bounce, with this 67 us; the frame 2.37 -> 1.19 ms.
+// took 211 us a bounce, with this 67 us; device time of the frame 2.37 ->
+// 1.19 ms.
 template <bool QUERY>
 __device__ __forceinline__ void block_append(unsigned long long* pair, uint32_t* qcount, bool next, bool shadow,
                                              bool query, uint32_t& inext, uint32_t& ishadow, uint32_t& iquery) {
