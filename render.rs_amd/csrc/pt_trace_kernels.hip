@@ -57,7 +57,6 @@ __global__ __launch_bounds__(kTraceBlock) void shadow_kernel(PtSceneView S, Path
 // ends with the few waves that hold its longest rays, so the shadow rays run
 // under the closest hits' end instead of after it. Extension rays, the
 // longer ones, come first. A wave's lanes all hold the same kind of ray.
-// Without a queue (q null) only the shadow records are traced.
 // With the counter rotation's launch gone as well, device time a frame: 540p
 // instanced field 18.6 -> 16.1 ms, 200 x 200 cloud room 4.46 -> 3.88, 256 x
 // 256 box room 1.08 -> 1.02.
@@ -66,7 +65,7 @@ __global__ __launch_bounds__(kTraceBlock) void trace_kernel(PtSceneView S, PathB
   constexpr int SG = GEO & ~kGeoSt;  // shadow rays need no texture coordinates
   __shared__ uint32_t s_stack[STACK * kTraceBlock];
   uint32_t* stk = s_stack + threadIdx.x;
-  const uint32_t live = q ? P.live() : 0, first = (live + 63u) & ~63u, n = first + P.shadows();
+  const uint32_t live = P.live(), first = (live + 63u) & ~63u, n = first + P.shadows();
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     if (i >= first)
@@ -88,11 +87,10 @@ void launch_trace_counted(const PtSceneView& S, const PathBuffers& P, const uint
     hipLaunchKernelGGL((shadow_kernel<STACK, true, MOTION, GEO, COUNT>), dim3(gt), dim3(kTraceBlock), 0, st, S, P);
   else if (S.transparent)
     hipLaunchKernelGGL((shadow_kernel<STACK, true, MOTION, SG, COUNT>), dim3(gt), dim3(kTraceBlock), 0, st, S, P);
-  else if constexpr (COUNT)
-    hipLaunchKernelGGL((shadow_kernel<STACK, false, MOTION, SG, COUNT>), dim3(gt), dim3(kTraceBlock), 0, st, S, P);
+  else if (work == kTraceRound)
+    hipLaunchKernelGGL((trace_kernel<STACK, MOTION, GEO>), dim3(gt), dim3(kTraceBlock), 0, st, S, P, q);
   else
-    hipLaunchKernelGGL((trace_kernel<STACK, MOTION, GEO>), dim3(gt), dim3(kTraceBlock), 0, st, S, P,
-                       work == kTraceRound ? q : nullptr);
+    hipLaunchKernelGGL((shadow_kernel<STACK, false, MOTION, SG, COUNT>), dim3(gt), dim3(kTraceBlock), 0, st, S, P);
 }
 
 template <int STACK, bool MOTION, int GEO>
